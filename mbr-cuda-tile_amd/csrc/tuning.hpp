@@ -36,6 +36,9 @@
 #ifndef MBRT_NT_ROW
 #define MBRT_NT_ROW 3    // row copy (permutes that keep the innermost dim)
 #endif
+#ifndef MBRT_NT_CAT
+#define MBRT_NT_CAT 2    // concat of several sources in one launch
+#endif
 #ifndef MBRT_NT_TR
 #define MBRT_NT_TR 0     // LDS tile transpose
 #endif

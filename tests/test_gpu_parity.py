@@ -105,6 +105,35 @@ def test_index_select_pad_cat(orc, dev):
     assert_bitexact(to_host(out, F32), np.concatenate(parts, axis=1), "cat")
 
 
+# (rows before the concat dim, source extents, elements after it, dtype, first-element offset of
+# the sources and the output): one column block, several, a row of columns just past one, more
+# sources than one launch holds, empty sources, every vector width, one row and many
+@pytest.mark.parametrize("outer,sizes,inner,dt,shift", [
+    (801, (28, 24, 24, 40, 520, 396), 1, F32, 0), (9, (257, 1, 3), 4, F32, 0), (1, (5000, 3, 70000), 1, F32, 0),
+    (17, tuple(4 * (1 + i % 7) for i in range(131)), 1, F32, 0), (33, (3, 0, 5, 0), 2, BF16, 0),
+    (7, (28, 24), 2, BF16, 0), (65, (1, 1), 1, BF16, 1), (40, (4, 8), 1, F32, 1), (3, (6, 2, 2), 3, I64, 0),
+    (2049, (1, 2), 1, F32, 0), (5, (64,) * 65, 8, F16, 4)])
+def test_cat_one_launch(orc, dev, outer, sizes, inner, dt, shift):
+    say(f"cat outer={outer} sizes={sizes[:4]}x{len(sizes)} inner={inner} dt={dt} shift={shift}")
+    rng = np.random.default_rng(outer * 31 + len(sizes))
+    npdt = {F32: np.float32, BF16: np.uint16, F16: np.uint16, I64: np.int64}[dt]
+
+    def shifted(n):  # n elements starting `shift` elements into an aligned buffer
+        return empty((n + shift,), dt)[shift:]
+
+    parts, devs = [], []
+    for n in sizes:
+        p = rng.integers(0, 2**15, size=(outer, n, inner)).astype(npdt)
+        d = shifted(p.size).view(outer, n, inner)
+        d.copy_(to_dev(p, dt))
+        parts.append(p)
+        devs.append(d)
+    out = shifted(outer * sum(sizes) * inner).view(outer, sum(sizes), inner)
+    mbrt.cat(devs, 1, out)
+    torch.cuda.synchronize()
+    assert_bitexact(to_host(out, dt), np.concatenate(parts, axis=1), "cat")
+
+
 # ---- element-wise ----------------------------------------------------------------------------
 
 @pytest.mark.parametrize("n", [0, 1, 7, 8, 1000, 4099])
