@@ -3,6 +3,7 @@
 Outputs (git-ignored, shipped with the source tree):
   mbr-cuda-tile_amd/lib/libmbrt.so        C-ABI + HIP kernels (include/mbrt.h)
   mbr-cuda-tile_amd/lib/libmbrt_tensor.so C++ Tensor / tensor_tile:: / mbr_tile:: layer
+  mbr-cuda-tile_amd/lib/_mbrt_calls.so    native calls of the Python binding (pyext/)
 
 Usage: python mbr-cuda-tile_amd/build.py [-j N] [-v] [-D NAME=VALUE ...] [--out DIR]
 
@@ -14,16 +15,19 @@ from __future__ import annotations
 
 import argparse
 import concurrent.futures as cf
+import importlib.util
 import os
 import shlex
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 REPO = PKG.parent
 CSRC = PKG / "csrc"
 HOST = PKG / "host"
+PYEXT = PKG / "pyext"
 BUILD = PKG / "_build"
 LIB = PKG / "lib"
 
@@ -121,20 +125,46 @@ def _objects(srcdir: Path, names: list[str], tag: str, build_dir: Path, defines:
     return objs
 
 
+def _compile_calls(build_dir: Path, verbose: bool) -> Path:
+    """The binding's extension module: host code against torch's and Python's headers."""
+    torch_dir = Path(importlib.util.find_spec("torch").submodule_search_locations[0])
+    obj = build_dir / "p_calls.o"
+    _run([HIPCC, "-x", "c++", "-O2", "-fPIC", "-fvisibility=hidden", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1",
+          "-DUSE_ROCM", f"-I{REPO / 'include'}", "-isystem", str(torch_dir / "include"), "-isystem",
+          str(torch_dir / "include" / "torch" / "csrc" / "api" / "include"), "-isystem",
+          sysconfig.get_paths()["include"], "-isystem", "/opt/rocm/include", "-c", str(PYEXT / "calls.cpp"), "-o",
+          str(obj)], verbose)
+    return obj
+
+
+def _link_calls(obj: Path, lib_dir: Path, verbose: bool) -> Path:
+    """torch's libraries are loaded before the module is, by the package's `import torch`."""
+    torch_lib = Path(importlib.util.find_spec("torch").submodule_search_locations[0]) / "lib"
+    ext = lib_dir / "_mbrt_calls.so"
+    tmp = ext.with_suffix(".so.tmp")
+    _run([HIPCC, "-shared", "-fPIC", "-o", str(tmp), str(obj), f"-L{lib_dir}", "-lmbrt", f"-L{torch_lib}",
+          "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"], verbose)
+    os.replace(tmp, ext)
+    return ext
+
+
 def build(jobs: int | None = None, verbose: bool = False, defines: list[str] | None = None,
           out_dir: Path | str | None = None) -> dict[str, Path]:
-    """Compile every source and link both libraries; returns their paths."""
+    """Compile every source and link the libraries and the extension module; returns their paths."""
     jobs = jobs or min(8, os.cpu_count() or 4)
     defines = list(defines or [])
     lib_dir = Path(out_dir) if out_dir else LIB
     build_dir = lib_dir / "_build" if out_dir else BUILD
     lib_dir.mkdir(parents=True, exist_ok=True)
-    kobjs = _objects(CSRC, KERNEL_SOURCES, "k", build_dir, defines, jobs, verbose)
+    build_dir.mkdir(parents=True, exist_ok=True)
+    with cf.ThreadPoolExecutor(max_workers=1) as ex:
+        calls_obj = ex.submit(_compile_calls, build_dir, verbose)  # beside the kernels
+        kobjs = _objects(CSRC, KERNEL_SOURCES, "k", build_dir, defines, jobs, verbose)
     libmbrt = lib_dir / "libmbrt.so"
     tmp = libmbrt.with_suffix(".so.tmp")
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, kobjs)], verbose)
     os.replace(tmp, libmbrt)
-    out = {"libmbrt": libmbrt}
+    out = {"libmbrt": libmbrt, "mbrt_calls": _link_calls(calls_obj.result(), lib_dir, verbose)}
     tsrc = [n for n in TENSOR_SOURCES if (HOST / n).exists()]
     if tsrc:
         tobjs = _objects(HOST, tsrc, "t", build_dir, defines, jobs, verbose)

@@ -1,7 +1,9 @@
 """Python binding of the mbrt C-ABI (include/mbrt.h) over torch device tensors.
 
 torch provides device memory and the stream only; every computation is a call into
-lib/libmbrt.so.  Each function enqueues on torch's current HIP stream (or `stream`).
+lib/libmbrt.so.  Each function enqueues on torch's current HIP stream (or `stream`).  The
+calls a model makes many times per chunk go through lib/_mbrt_calls.so (pyext/calls.cpp),
+which reads the tensors natively; the others through ctypes.
 """
 from __future__ import annotations
 
@@ -28,10 +30,14 @@ def dtype_code(t: torch.Tensor) -> int:
         raise TypeError(f"mbrt: unsupported dtype {t.dtype}") from e
 
 
+def _stream_handle(stream) -> int:
+    return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
+
+
 def _s(stream) -> C.c_void_p:
     if stream is None:
         stream = torch.cuda.current_stream()
-    return C.c_void_p(stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream))
+    return C.c_void_p(_stream_handle(stream))
 
 
 def _p(t: torch.Tensor | None) -> C.c_void_p:
@@ -42,6 +48,23 @@ def _contig(*ts: torch.Tensor) -> None:
     for t in ts:
         if t is not None and not t.is_contiguous():
             raise ValueError("mbrt: expected a contiguous tensor")
+
+
+class _Native:
+    """Stands for the native calls until the first one, then loads them in its place."""
+
+    def __getattr__(self, name):
+        global _n
+        _n = _abi.load_calls()
+        return getattr(_n, name)
+
+
+_n = _Native()
+
+
+def _h(stream) -> int | None:
+    """A stream argument for a native call: None is torch's current stream."""
+    return None if stream is None else _stream_handle(stream)
 
 
 def version() -> int:
@@ -81,8 +104,7 @@ class arith_flags:
 # ---- tensor library --------------------------------------------------------------------
 
 def fill_(t: torch.Tensor, value: float, stream=None) -> torch.Tensor:
-    _contig(t)
-    _abi.call("mbrt_fill", _p(t), dtype_code(t), t.numel(), float(value), _s(stream))
+    _n.fill(t, value, _h(stream))
     return t
 
 
@@ -154,11 +176,7 @@ def strided_meta(shape: Sequence[int], strides: Sequence[int]) -> _abi.StridedMe
 
 def strided_copy(src: torch.Tensor, dst: torch.Tensor, stream=None) -> torch.Tensor:
     """dst (contiguous) = src (any strided view), e.g. x.permute(...) -> contiguous."""
-    _contig(dst)
-    if list(dst.shape) != list(src.shape):
-        raise ValueError("strided_copy: shape mismatch")
-    m = strided_meta(src.shape, src.stride())
-    _abi.call("mbrt_strided_copy", _p(src), _p(dst), dtype_code(src), C.byref(m), _s(stream))
+    _n.strided_copy(src, dst, _h(stream))
     return dst
 
 
@@ -173,37 +191,12 @@ def index_select(src: torch.Tensor, dim: int, idx: torch.Tensor, out: torch.Tens
 
 def pad(src: torch.Tensor, out: torch.Tensor, before: Sequence[int], value: float = 0.0, reflect: bool = False,
         stream=None) -> torch.Tensor:
-    _contig(src, out)
-    m = _abi.PadMeta()
-    m.ndim = src.dim()
-    for d in range(src.dim()):
-        m.src_shape[d] = src.shape[d]
-        m.dst_shape[d] = out.shape[d]
-        m.pad_before[d] = before[d]
-    if reflect:
-        _abi.call("mbrt_pad_reflect", _p(src), _p(out), dtype_code(src), C.byref(m), _s(stream))
-    else:
-        _abi.call("mbrt_pad_const", _p(src), _p(out), dtype_code(src), C.byref(m), float(value), _s(stream))
+    _n.pad(src, out, before, value, reflect, _h(stream))
     return out
 
 
 def cat(srcs: Sequence[torch.Tensor], dim: int, out: torch.Tensor, stream=None) -> torch.Tensor:
-    _contig(out, *srcs)
-    dim = dim % out.dim()
-    outer = 1
-    for d in range(dim):
-        outer *= out.shape[d]
-    inner = 1
-    for d in range(dim + 1, out.dim()):
-        inner *= out.shape[d]
-    arr = (_abi.CatSrc * len(srcs))()
-    off = 0
-    for i, s in enumerate(srcs):
-        arr[i].ptr = s.data_ptr()
-        arr[i].dim_size = s.shape[dim]
-        arr[i].dim_offset = off
-        off += s.shape[dim]
-    _abi.call("mbrt_cat", _p(out), arr, len(srcs), outer, out.shape[dim], inner * out.element_size(), _s(stream))
+    _n.cat(srcs, dim, out, _h(stream))
     return out
 
 
@@ -232,61 +225,36 @@ def reduce_general(src: torch.Tensor, dst: torch.Tensor, dim: int, op: int, stre
 
 def rms_norm(x: torch.Tensor, gamma: torch.Tensor, out: torch.Tensor, scale: float, eps: float = 1e-12,
              stream=None) -> torch.Tensor:
-    _contig(x, gamma, out)
-    dim = x.shape[-1]
-    _abi.call("mbrt_rms_norm", _p(x), dtype_code(x), _p(gamma), dtype_code(gamma), _p(out), dtype_code(out),
-              x.numel() // dim, dim, scale, eps, _s(stream))
+    _n.rms_norm(x, gamma, out, scale, eps, _h(stream))
     return out
 
 
 def residual_add_rms_norm(residual: torch.Tensor, update: torch.Tensor, gamma: torch.Tensor,
                           sum_out: torch.Tensor | None, normed: torch.Tensor, scale: float, eps: float = 1e-12,
                           stream=None) -> torch.Tensor:
-    _contig(residual, update, gamma, sum_out, normed)
-    dim = residual.shape[-1]
-    sdt = dtype_code(sum_out) if sum_out is not None else dtype_code(residual)
-    _abi.call("mbrt_residual_add_rms_norm", _p(residual), _p(update), dtype_code(residual), _p(gamma),
-              dtype_code(gamma), _p(sum_out), sdt, _p(normed), dtype_code(normed), residual.numel() // dim, dim,
-              scale, eps, _s(stream))
+    _n.residual_add_rms_norm(residual, update, gamma, sum_out, normed, scale, eps, _h(stream))
     return normed
 
 
 def bias_act(x: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor, act: int, stream=None) -> torch.Tensor:
-    _contig(x, bias, out)
-    cols = x.shape[-1]
-    _abi.call("mbrt_bias_act", _p(x), dtype_code(x), _p(bias), dtype_code(bias) if bias is not None else F32, _p(out),
-              dtype_code(out), x.numel() // cols, cols, act, _s(stream))
+    _n.bias_act(x, bias, out, act, _h(stream))
     return out
 
 
 def glu(x: torch.Tensor, out: torch.Tensor, stream=None) -> torch.Tensor:
-    _contig(x, out)
-    full = x.shape[-1]
-    if full % 2:
-        raise ValueError("glu_last_dim: last dimension must be even")
-    _abi.call("mbrt_glu_last_dim", _p(x), dtype_code(x), _p(out), dtype_code(out), x.numel() // full, full // 2,
-              _s(stream))
+    _n.glu(x, out, _h(stream))
     return out
 
 
 def gate_merge(attn: torch.Tensor, gate: torch.Tensor, out: torch.Tensor, layout: int = LAYOUT_BHND,
                gate_is_logit: bool = True, stream=None) -> torch.Tensor:
     """attn [B,H,N,D] (BHND) or [B,N,H,D] (BNHD); gate [B,N,H]; out [B,N,H*D]."""
-    _contig(attn, gate, out)
-    if layout == LAYOUT_BHND:
-        B, H, N, D = attn.shape
-    else:
-        B, N, H, D = attn.shape
-    _abi.call("mbrt_sigmoid_gate_merge", _p(attn), dtype_code(attn), _p(gate), dtype_code(gate),
-              1 if gate_is_logit else 0, _p(out), dtype_code(out), B, H, N, D, layout, _s(stream))
+    _n.gate_merge(attn, gate, out, layout, gate_is_logit, _h(stream))
     return out
 
 
 def softmax(x: torch.Tensor, out: torch.Tensor, scale: float = 1.0, stream=None) -> torch.Tensor:
-    _contig(x, out)
-    cols = x.shape[-1]
-    _abi.call("mbrt_softmax_rows", _p(x), dtype_code(x), _p(out), dtype_code(out), x.numel() // cols, cols, scale,
-              _s(stream))
+    _n.softmax(x, out, scale, _h(stream))
     return out
 
 
@@ -302,12 +270,7 @@ def rotary_(q: torch.Tensor, k: torch.Tensor | None, cos: torch.Tensor, sin: tor
 
 def split_qkv_rotary(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, q: torch.Tensor, k: torch.Tensor,
                      v: torch.Tensor, heads: int, stream=None) -> None:
-    _contig(qkv, cos, sin, q, k, v)
-    B, N, three_hd = qkv.shape
-    D = three_hd // (3 * heads)
-    out_n = q.shape[2]
-    _abi.call("mbrt_split_qkv_heads_rotary", _p(qkv), dtype_code(qkv), _p(cos), _p(sin), dtype_code(cos), _p(q),
-              _p(k), _p(v), dtype_code(q), B, N, heads, D, out_n, _s(stream))
+    _n.split_qkv_rotary(qkv, cos, sin, q, k, v, heads, _h(stream))
 
 
 def band_gather(stft: torch.Tensor, idx: torch.Tensor, out: torch.Tensor, stream=None) -> torch.Tensor:
@@ -361,14 +324,8 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tens
         _contig(t)
     BH, nq, D = q.shape
     nk = k.shape[1]
-    pm = _p_precision(p_bf16, p_precision)
-    if pm == ATTN_P_PAIR:
-        _abi.call("mbrt_attention", _p(q), _p(k), _p(v), dtype_code(q), _p(out), dtype_code(out), BH, nq, nk, D,
-                  float(scale), _s(stream))
-    else:
-        _abi.call("mbrt_attention_ex", _p(q), _p(k), _p(v), dtype_code(q), BH, 1, nq, nk, D, nq * D, 0, D,
-                  nk * D, 0, D, None, None, F32, None, F32, 0, _p(out), dtype_code(out), float(scale),
-                  pm, _s(stream))
+    _n.attention_ex(q, k, v, (BH, 1, nq, nk, D), (nq * D, 0, D, nk * D, 0, D), None, None, None, 0, out, scale,
+                    _p_precision(p_bf16, p_precision), _h(stream))
     return out
 
 
@@ -394,13 +351,9 @@ def attention_bnhd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch
     for t in (cos, sin, gate):
         if t is not None:
             _contig(t)
-    _abi.call("mbrt_attention_ex", _p(q), _p(k), _p(v), dtype_code(q), B, H, nq, nk, D,
-              q.stride(0), q.stride(2), q.stride(1), k.stride(0), k.stride(2), k.stride(1),
-              _p(cos) if cos is not None else None, _p(sin) if sin is not None else None,
-              dtype_code(cos) if cos is not None else F32,
-              _p(gate) if gate is not None else None, dtype_code(gate) if gate is not None else F32,
-              int(gate_is_logit), _p(out), dtype_code(out), float(scale), _p_precision(p_bf16, p_precision),
-              _s(stream))
+    _n.attention_ex(q, k, v, (B, H, nq, nk, D),
+                    (q.stride(0), q.stride(2), q.stride(1), k.stride(0), k.stride(2), k.stride(1)), cos, sin, gate,
+                    gate_is_logit, out, scale, _p_precision(p_bf16, p_precision), _h(stream))
     return out
 
 
@@ -429,9 +382,7 @@ def stft(signal: torch.Tensor, window: torch.Tensor, hop: int, center: bool = Tr
     T = stft_num_frames(L, hop, center)
     if out is None:
         out = torch.empty((B, n_fft // 2 + 1, max(T, 0), 2), dtype=torch.float32, device=x.device)
-    _contig(out)
-    _abi.call("mbrt_stft", _p(x), _p(window), _p(out), B, L, n_fft, hop, win_length, window.numel(), int(center),
-              int(normalized), _s(stream))
+    _n.stft(x, window, hop, center, normalized, out, n_fft, win_length, _h(stream))
     return out
 
 
@@ -453,12 +404,10 @@ def istft(spec: torch.Tensor, window: torch.Tensor, hop: int, center: bool = Tru
     if out is None:
         out = torch.empty((B, max(n_out, 0)), dtype=torch.float32, device=spec.device)
     _contig(out)
-    need = int(_abi.lib().mbrt_istft_workspace_bytes(B, T, hop))
     if workspace is None:
+        need = istft_workspace_bytes(B, T, hop)
         workspace = torch.empty(max(need, 0) // 4, dtype=torch.float32, device=spec.device)
-    _abi.call("mbrt_istft", _p(spec), dtype_code(spec), _p(window), _p(out), B, F, T, n_fft, hop, win_length,
-              window.numel(), int(center), int(normalized), length, _p(workspace),
-              workspace.numel() * workspace.element_size(), _s(stream))
+    _n.istft(spec, window, hop, center, normalized, length, out, workspace, n_fft, win_length, _h(stream))
     return out
 
 
@@ -480,10 +429,7 @@ def istft_noalloc(spec: torch.Tensor, window: torch.Tensor, hop: int, out: torch
 def chunk_accumulate(dest: torch.Tensor, weight_sum: torch.Tensor, src: torch.Tensor, window: torch.Tensor,
                      offset: int, stream=None) -> torch.Tensor:
     """dest [.., L] += src [.., n] * window at `offset` (channels = src.numel() / n); weight_sum += window."""
-    _contig(dest, weight_sum, src, window)
-    n, L = src.shape[-1], dest.shape[-1]
-    _abi.call("mbrt_chunk_accumulate", _p(dest), _p(weight_sum), _p(src), _p(window), src.numel() // max(n, 1), n, L,
-              offset, _s(stream))
+    _n.chunk_accumulate(dest, weight_sum, src, window, offset, _h(stream))
     return dest
 
 

@@ -6,10 +6,12 @@ library is missing, importing raises (build it with `python mbr-cuda-tile_amd/bu
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent.parent
 LIB_PATH = PKG_DIR / "lib" / "libmbrt.so"
+CALLS_PATH = PKG_DIR / "lib" / "_mbrt_calls.so"
 
 MAX_DIMS = 8
 
@@ -151,6 +153,18 @@ def lib() -> C.CDLL:
     if _LIB is None:
         _LIB = load()
     return _LIB
+
+
+def load_calls(path: Path | str = CALLS_PATH):
+    """The extension module of native calls (pyext/calls.cpp); it links libmbrt.so."""
+    path = Path(path)
+    if not path.exists():
+        raise ImportError(f"mbrt: {path} is not built (run python mbr-cuda-tile_amd/build.py)")
+    spec = importlib.util.spec_from_file_location("_mbrt_calls", path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    mod.init(MbrtError)
+    return mod
 
 
 def call(name: str, *args) -> None:

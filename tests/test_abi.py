@@ -231,3 +231,34 @@ def test_last_error_is_per_thread(lib):
         t.join()
     assert len(seen["glu"]) == 1 and len(seen["rotary"]) == 1
     assert seen["glu"] != seen["rotary"] and all("even" in m for m in seen["rotary"])
+
+
+def test_native_calls_refuse_what_the_binding_documents(lib):
+    """The binding's native calls (pyext/calls.cpp) check their tensors before anything is launched:
+    CPU tensors and stream 0 stand in, no call gets as far as the GPU."""
+    import torch
+
+    import mbrt
+
+    x, y = torch.empty(4, 8), torch.empty(4, 8)
+    for exc, match, fn in [
+        (ValueError, "contiguous", lambda: mbrt.rms_norm(x.t(), x[0], y, 1.0, stream=0)),
+        (ValueError, "contiguous", lambda: mbrt.chunk_accumulate(x, x[0], y.t(), y[0], 0, stream=0)),
+        (ValueError, "even", lambda: mbrt.glu(torch.empty(4, 7), y, stream=0)),
+        (ValueError, "shape mismatch", lambda: mbrt.strided_copy(x, torch.empty(3, 8), stream=0)),
+        (ValueError, "4-d", lambda: mbrt.gate_merge(x, x, y, stream=0)),
+        (TypeError, "torch.bool", lambda: mbrt.softmax(x.bool(), y, stream=0)),
+        (TypeError, "Tensor", lambda: mbrt.softmax(1, y, stream=0)),
+        (TypeError, "Tensor", lambda: mbrt.cat([x, None], 0, y, stream=0)),
+        (TypeError, "", lambda: mbrt.softmax(x, y, "a", stream=0)),
+        (ZeroDivisionError, "", lambda: mbrt.rms_norm(torch.empty(4, 0), x[0], y, 1.0, stream=0)),
+        (IndexError, "", lambda: mbrt.softmax(torch.tensor(1.0), y, stream=0)),
+    ]:
+        with pytest.raises(exc, match=match):
+            fn()
+    with pytest.raises(mbrt.MbrtError, match="mbrt_softmax_rows -> MBRT_E_UNSUPPORTED_DTYPE.*dtype 2") as e:
+        mbrt.softmax(x.long(), y, stream=0)
+    assert e.value.status == 2
+    assert mbrt.fill_(torch.empty(0), 1.0, stream=0).numel() == 0  # nothing to do: no launch
+    with pytest.raises(mbrt.MbrtError, match="SHAPE"):
+        mbrt.chunk_accumulate(x, x[0], y, y[0], 5, stream=0)
