@@ -352,6 +352,25 @@ __device__ __forceinline__ void gst(T* p, T v) {
     else *p = v;
 }
 
+// 16 bytes at an address aligned to A bytes only (A = 4 or 2): one dwordx4 access, which
+// global memory takes at any alignment (unaligned access mode, the default of HSA code).
+template <int A>
+struct AnyVec;
+template <> struct AnyVec<4> { typedef uint32_t T __attribute__((ext_vector_type(4), aligned(4))); };
+template <> struct AnyVec<2> { typedef uint32_t T __attribute__((ext_vector_type(4), aligned(2))); };
+template <int NT, int A>
+__device__ __forceinline__ u32x4 ld_any(const void* p) {
+    typedef typename AnyVec<A>::T W;
+    if constexpr ((NT & 1) != 0) return __builtin_nontemporal_load(reinterpret_cast<const W*>(p));
+    else return *reinterpret_cast<const W*>(p);
+}
+template <int NT, int A>
+__device__ __forceinline__ void st_any(void* p, u32x4 v) {
+    typedef typename AnyVec<A>::T W;
+    if constexpr ((NT & 2) != 0) __builtin_nontemporal_store(v, reinterpret_cast<W*>(p));
+    else *reinterpret_cast<W*>(p) = v;
+}
+
 template <int DT>
 struct DtSize {
     static constexpr int value = DT == F32 ? 4 : 2;

@@ -10,25 +10,27 @@
 // reference's atomic add of a rounded product is).
 //
 // Memory-bound: per call C*n reads of src, C*n read-modify-writes of dest, n of the window
-// and n read-modify-writes of the weight sum.  A thread owns one sample position (or four)
-// and walks a group of channels (all channels for the normalize), so the window and the
-// weight sum are not re-read per channel.  16-byte vectors when the offset, lengths and
-// pointers allow, else a scalar path.
+// and n read-modify-writes of the weight sum.  A thread owns four sample positions
+// (of one channel, or of all channels for the normalize).  16-byte accesses at any sample
+// alignment: a song of odd length puts its second channel, and a chunk at an odd offset all of
+// its rows, off 16-byte addresses.  Per-sample kernels for those took 5.68 us per chunk of
+// [2, 352800] and 13.1 us to normalize [2, 2997817]; these take 4.9 and 12.1.
 #include "abi_common.hpp"
 
 namespace mbrt {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-// float4 through the non-temporal load / store helpers (which take ext-vector types)
+// 4 floats at any float address through the vector helpers
+struct F4 {
+    float v[4];
+};
 template <int NT>
-__device__ __forceinline__ float4 ld4(const float4* p) {
-    const f32x4 v = gld<NT>(reinterpret_cast<const f32x4*>(p));
-    return make_float4(v.x, v.y, v.z, v.w);
+__device__ __forceinline__ F4 ld4(const float* p) {
+    return __builtin_bit_cast(F4, ld_any<NT, 4>(p));
 }
 template <int NT>
-__device__ __forceinline__ void st4(float4* p, float4 v) {
-    gst<NT>(reinterpret_cast<f32x4*>(p), f32x4{v.x, v.y, v.z, v.w});
+__device__ __forceinline__ void st4(float* p, const F4& x) {
+    st_any<NT, 4>(p, __builtin_bit_cast(u32x4, x));
 }
 
 constexpr int kThreads = 256;
@@ -38,7 +40,7 @@ struct AccArgs {
     float* __restrict__ wsum;       // [dest_len]
     const float* __restrict__ src;  // [C, n]
     const float* __restrict__ win;  // [n]
-    int64_t n;            // chunk length (elements, or 4-element vectors on the vector path)
+    int64_t n;            // chunk length
     int64_t dest_len;
     int64_t offset;
     int64_t channels;
@@ -50,79 +52,40 @@ __device__ __forceinline__ float acc1(float d, float s, float w) {
     return d + s * w;
 }
 
-// grid: x over the chunk (grid-stride), y over groups of kCG channels; a thread walks the
-// channels of its group, so the window is read once per group and the weight sum once
-constexpr int kCG = 1;  // measured: 1 (11.7 us) beats 4 (12.4 us) and all channels (12.8 us) at 8 x 352800
-
-__global__ __launch_bounds__(kThreads) void accumulate_scalar_kernel(AccArgs a) {
-    const int64_t c0 = (int64_t)blockIdx.y * kCG, c1 = min(c0 + kCG, a.channels);
-    for (int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x; k < a.n; k += (int64_t)gridDim.x * kThreads) {
-        const float w = a.win[k];
-        for (int64_t c = c0; c < c1; ++c) {
-            float* d = a.dest + c * a.dest_len + a.offset + k;
-            *d = acc1(*d, a.src[c * a.n + k], w);
-        }
-        if (blockIdx.y == 0) a.wsum[a.offset + k] = a.wsum[a.offset + k] + w;
-    }
-}
-
-// n, dest_len and offset in float4 units
-__global__ __launch_bounds__(kThreads) void accumulate_vec_kernel(AccArgs a) {
-    const int64_t c0 = (int64_t)blockIdx.y * kCG, c1 = min(c0 + kCG, a.channels);
-    for (int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x; k < a.n; k += (int64_t)gridDim.x * kThreads) {
-        const float4 w = reinterpret_cast<const float4*>(a.win)[k];
-#pragma unroll
-        for (int u = 0; u < kCG; ++u) {
-            const int64_t c = c0 + u;
-            if (c >= c1) break;
-            const float4 s = reinterpret_cast<const float4*>(a.src)[c * a.n + k];
-            float4* dp = reinterpret_cast<float4*>(a.dest) + c * a.dest_len + a.offset + k;
-            float4 d = *dp;
-            d.x = acc1(d.x, s.x, w.x);
-            d.y = acc1(d.y, s.y, w.y);
-            d.z = acc1(d.z, s.z, w.z);
-            d.w = acc1(d.w, s.w, w.w);
-            *dp = d;
-        }
-        if (blockIdx.y == 0) {
-            float4* wp = reinterpret_cast<float4*>(a.wsum) + a.offset + k;
-            float4 ws = *wp;
-            ws.x = ws.x + w.x;
-            ws.y = ws.y + w.y;
-            ws.z = ws.z + w.z;
-            ws.w = ws.w + w.w;
-            *wp = ws;
-        }
-    }
-}
-
 // One wave per channel: a block of CPB waves takes channels [CPB y, CPB y + CPB) over the
-// same 64 consecutive float4 positions of the chunk, so the window's repeated reads are
-// made by waves of one CU, close together in time (float4 units as above).
+// same 64 consecutive 4-sample positions of the chunk, so the window's repeated reads are
+// made by waves of one CU, close together in time.  Positions are vectors of the chunk
+// (the last one may hold fewer than 4 samples): dest, weight sum and window addresses are
+// only sample-aligned where a song's length or a chunk's offset is odd, and 16-byte accesses
+// take that (ld_any).
 template <int CPB>
 __global__ __launch_bounds__(64 * CPB) void accumulate_cw_kernel(AccArgs a) {
     const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
     const int64_t c = (int64_t)blockIdx.y * CPB + w;
-    for (int64_t k = (int64_t)blockIdx.x * 64 + lane; k < a.n; k += (int64_t)gridDim.x * 64) {
-        const float4 wv = reinterpret_cast<const float4*>(a.win)[k];
-        if (c < a.channels) {
-            const float4 s = ld4<MBRT_NT_CHUNK & 1>(reinterpret_cast<const float4*>(a.src) + c * a.n + k);
-            float4* dp = reinterpret_cast<float4*>(a.dest) + c * a.dest_len + a.offset + k;
-            float4 d = ld4<MBRT_NT_CHUNK & 1>(dp);
-            d.x = acc1(d.x, s.x, wv.x);
-            d.y = acc1(d.y, s.y, wv.y);
-            d.z = acc1(d.z, s.z, wv.z);
-            d.w = acc1(d.w, s.w, wv.w);
+    const bool wsum = blockIdx.y == 0 && w == 0;
+    if (c >= a.channels) return;
+    for (int64_t k = 4 * ((int64_t)blockIdx.x * 64 + lane); k < a.n; k += 4 * (int64_t)gridDim.x * 64) {
+        const float* sp = a.src + c * a.n + k;
+        float* dp = a.dest + c * a.dest_len + a.offset + k;
+        float* wp = a.wsum + a.offset + k;
+        if (k + 4 <= a.n) {
+            const F4 wv = ld4<0>(a.win + k);
+            const F4 s = ld4<MBRT_NT_CHUNK & 1>(sp);
+            F4 d = ld4<MBRT_NT_CHUNK & 1>(dp);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d.v[e] = acc1(d.v[e], s.v[e], wv.v[e]);
             st4<MBRT_NT_CHUNK & 2>(dp, d);
-        }
-        if (blockIdx.y == 0 && w == 0) {
-            float4* wp = reinterpret_cast<float4*>(a.wsum) + a.offset + k;
-            float4 ws = *wp;
-            ws.x = ws.x + wv.x;
-            ws.y = ws.y + wv.y;
-            ws.z = ws.z + wv.z;
-            ws.w = ws.w + wv.w;
-            *wp = ws;
+            if (wsum) {
+                F4 ws = ld4<0>(wp);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ws.v[e] = ws.v[e] + wv.v[e];
+                st4<0>(wp, ws);
+            }
+        } else {
+            for (int e = 0; e < (int)(a.n - k); ++e) {
+                dp[e] = acc1(dp[e], sp[e], a.win[k + e]);
+                if (wsum) wp[e] = wp[e] + a.win[k + e];
+            }
         }
     }
 }
@@ -130,31 +93,31 @@ __global__ __launch_bounds__(64 * CPB) void accumulate_cw_kernel(AccArgs a) {
 struct NormArgs {
     float* __restrict__ data;        // [C, len]
     const float* __restrict__ wsum;  // [len]
-    int64_t len;          // elements, or float4 units on the vector path
+    int64_t len;
     int64_t channels;
 };
 
 __device__ __forceinline__ float norm1(float v, float w) { return w > 1.0e-8f ? v / w : v; }
 
-__global__ __launch_bounds__(kThreads) void normalize_scalar_kernel(NormArgs a) {
-    for (int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x; k < a.len; k += (int64_t)gridDim.x * kThreads) {
-        const float w = a.wsum[k];
-        for (int64_t c = 0; c < a.channels; ++c) a.data[c * a.len + k] = norm1(a.data[c * a.len + k], w);
-    }
-}
-
+// A thread owns 4 sample positions (the last one may hold fewer) and walks the channels, whose
+// rows are only sample-aligned where the length is not a multiple of 4.
 __global__ __launch_bounds__(kThreads) void normalize_vec_kernel(NormArgs a) {
-    for (int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x; k < a.len; k += (int64_t)gridDim.x * kThreads) {
-        const float4 w = reinterpret_cast<const float4*>(a.wsum)[k];
+    for (int64_t k = 4 * ((int64_t)blockIdx.x * kThreads + threadIdx.x); k < a.len;
+         k += 4 * (int64_t)gridDim.x * kThreads) {
+        if (k + 4 <= a.len) {
+            const F4 w = ld4<0>(a.wsum + k);
 #pragma unroll 4
-        for (int64_t c = 0; c < a.channels; ++c) {
-            float4* p = reinterpret_cast<float4*>(a.data) + c * a.len + k;
-            float4 v = ld4<MBRT_NT_CHUNK & 1>(p);
-            v.x = norm1(v.x, w.x);
-            v.y = norm1(v.y, w.y);
-            v.z = norm1(v.z, w.z);
-            v.w = norm1(v.w, w.w);
-            st4<MBRT_NT_CHUNK & 2>(p, v);
+            for (int64_t c = 0; c < a.channels; ++c) {
+                float* p = a.data + c * a.len + k;
+                F4 v = ld4<MBRT_NT_CHUNK & 1>(p);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v.v[e] = norm1(v.v[e], w.v[e]);
+                st4<MBRT_NT_CHUNK & 2>(p, v);
+            }
+        } else {
+            for (int e = 0; e < (int)(a.len - k); ++e)
+                for (int64_t c = 0; c < a.channels; ++c)
+                    a.data[c * a.len + k + e] = norm1(a.data[c * a.len + k + e], a.wsum[k + e]);
         }
     }
 }
@@ -178,26 +141,18 @@ int mbrt_chunk_accumulate(float* dest, float* weight_sum, const float* src, cons
     if (channels == 0 || chunk_len == 0) return MBRT_OK;
     MBRT_REQUIRE(dest && weight_sum && src && window, MBRT_E_INVALID_ARG, "%s: NULL pointer", op);
     AccArgs a{dest, weight_sum, src, window, chunk_len, dest_len, offset, channels};
-    const bool vec = chunk_len % 4 == 0 && dest_len % 4 == 0 && offset % 4 == 0 && aligned(dest, 16) &&
-                     aligned(weight_sum, 16) && aligned(src, 16) && aligned(window, 16);
     hipStream_t st = as_stream(stream);
-    const unsigned gy = (unsigned)std::min<int64_t>(ceil_div(channels, kCG), 65535);
-    MBRT_REQUIRE(channels <= (int64_t)kCG * 65535, MBRT_E_SHAPE, "%s: too many channels", op);
-    if (vec) {
-        a.n /= 4;
-        a.dest_len /= 4;
-        a.offset /= 4;
-        if (MBRT_CHUNK_CPB > 0) {
-            constexpr int CPB = MBRT_CHUNK_CPB > 0 ? MBRT_CHUNK_CPB : 1;
-            const unsigned gx = (unsigned)std::min<int64_t>(ceil_div(a.n, 64), int64_t(1) << 16);
-            hipLaunchKernelGGL(accumulate_cw_kernel<CPB>, dim3(gx, (unsigned)ceil_div(channels, CPB)), dim3(64 * CPB), 0,
-                               st, a);
-        } else {
-            hipLaunchKernelGGL(accumulate_vec_kernel, dim3((unsigned)grid_for(a.n), gy), dim3(kThreads), 0, st, a);
-        }
-    } else {
-        hipLaunchKernelGGL(accumulate_scalar_kernel, dim3((unsigned)grid_for(a.n), gy), dim3(kThreads), 0, st, a);
-    }
+    MBRT_REQUIRE(channels <= 65535, MBRT_E_SHAPE, "%s: too many channels", op);
+    auto launch = [&](auto cpb) {
+        constexpr int CPB = decltype(cpb)::value;
+        const unsigned gx = (unsigned)std::min<int64_t>(ceil_div(chunk_len, 256), int64_t(1) << 16);
+        hipLaunchKernelGGL(accumulate_cw_kernel<CPB>, dim3(gx, (unsigned)ceil_div(channels, CPB)), dim3(64 * CPB), 0, st,
+                           a);
+    };
+    // no more waves in a block than there are channels
+    if (channels <= 1) launch(std::integral_constant<int, 1>{});
+    else if (channels <= 2) launch(std::integral_constant<int, 2>{});
+    else launch(std::integral_constant<int, MBRT_CHUNK_CPB>{});
     return check_launch(op);
 }
 
@@ -208,14 +163,8 @@ int mbrt_chunk_normalize(float* data, const float* weight_sum, int64_t channels,
     if (channels == 0 || length == 0) return MBRT_OK;
     MBRT_REQUIRE(data && weight_sum, MBRT_E_INVALID_ARG, "%s: NULL pointer", op);
     NormArgs a{data, weight_sum, length, channels};
-    const bool vec = length % 4 == 0 && aligned(data, 16) && aligned(weight_sum, 16);
-    hipStream_t st = as_stream(stream);
-    if (vec) {
-        a.len /= 4;
-        hipLaunchKernelGGL(normalize_vec_kernel, dim3((unsigned)grid_for(a.len)), dim3(kThreads), 0, st, a);
-    } else {
-        hipLaunchKernelGGL(normalize_scalar_kernel, dim3((unsigned)grid_for(a.len)), dim3(kThreads), 0, st, a);
-    }
+    hipLaunchKernelGGL(normalize_vec_kernel, dim3((unsigned)grid_for(ceil_div(length, 4))), dim3(kThreads), 0,
+                       as_stream(stream), a);
     return check_launch(op);
 }
 

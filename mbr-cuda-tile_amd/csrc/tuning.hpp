@@ -36,6 +36,12 @@
 #ifndef MBRT_NT_ROW
 #define MBRT_NT_ROW 3    // row copy (permutes that keep the innermost dim)
 #endif
+#ifndef MBRT_NT_ROWU
+#define MBRT_NT_ROWU 2   // row copy of element-aligned rows in 16-byte vectors
+#endif
+#ifndef MBRT_ROWU_MIN
+#define MBRT_ROWU_MIN 64 // shortest such row, in bytes
+#endif
 #ifndef MBRT_NT_CAT
 #define MBRT_NT_CAT 2    // concat of several sources in one launch
 #endif
@@ -149,7 +155,7 @@
 #define MBRT_GATE_BPC 16  // sigmoid gate x head merge: blocks per CU of a grid that walks the chunks (0: one chunk per block)
 #endif
 #ifndef MBRT_CHUNK_CPB
-#define MBRT_CHUNK_CPB 4  // chunk accumulate: channels (one wave each) per block over shared positions (0: one channel per grid row)
+#define MBRT_CHUNK_CPB 4  // chunk accumulate: channels (one wave each) per block over shared positions (fewer when there are fewer channels)
 #endif
 #ifndef MBRT_EW_U
 #define MBRT_EW_U 4      // 16-byte groups per thread in the elementwise kernels

@@ -105,6 +105,48 @@ def test_index_select_pad_cat(orc, dev):
     assert_bitexact(to_host(out, F32), np.concatenate(parts, axis=1), "cat")
 
 
+# element-aligned rows around the shortest that go in 16-byte vectors (64 bytes), first
+# elements 0..3 past an aligned address, odd pitches, one row and many, a second outer dim
+@pytest.mark.parametrize("dt", [F32, BF16])
+@pytest.mark.parametrize("shape,n,start", [((5, 40), 15, 1), ((5, 40), 16, 1), ((5, 41), 17, 2), ((7, 81), 33, 3),
+                                           ((7, 80), 31, 0), ((3, 1003), 997, 1), ((1, 5001), 5000, 1),
+                                           ((2, 3, 4099), 4097, 2), ((300, 67), 66, 1)])
+def test_strided_copy_element_aligned_rows(orc, dev, dt, shape, n, start):
+    say(f"strided_copy rows of {n} from {start} of {shape} dt={dt}")
+    rng = np.random.default_rng(n * 7 + start)
+    x = rng.integers(0, 2**15, size=shape).astype(np.float32 if dt == F32 else np.uint16)
+    y = empty(tuple(shape[:-1]) + (n,), dt)
+    mbrt.strided_copy(to_dev(x, dt)[..., start:start + n], y)
+    torch.cuda.synchronize()
+    assert_bitexact(to_host(y, dt), np.ascontiguousarray(x[..., start:start + n]), "rows")
+
+
+# innermost-dim pads by whole rows: borders of 0 and up to the row (reflected) or past it, vectors
+# across both edges, sources of one element and shorter than a vector, cropping borders, a row
+# shorter than a vector (the general kernel)
+@pytest.mark.parametrize("dt", [F32, BF16, I64])
+@pytest.mark.parametrize("rows,n,before,m", [(2, 1001, 500, 2001), (3, 17, 3, 40), (1, 5, 4, 13), (2, 1, 2, 9), (4, 3, 0, 8),
+                                             (2, 100, 0, 100), (2, 100, 0, 131), (3, 64, 63, 190), (1, 30, -7, 16),
+                                             (2, 2, 1, 3), (1, 4000, 1777, 9001), (5, 33, 40, 120)])
+def test_pad_rows(orc, dev, dt, rows, n, before, m):
+    say(f"pad rows={rows} n={n} before={before} m={m} dt={dt}")
+    rng = np.random.default_rng(n * 13 + m)
+    x = rng.integers(1, 2**15, size=(rows, n)).astype({F32: np.float32, BF16: np.uint16, I64: np.int64}[dt])
+    c = np.arange(m) - before
+    for reflect in (False, True):
+        out = empty((rows, m), dt)
+        mbrt.pad(to_dev(x, dt), out, [0, before], value=2.0, reflect=reflect)
+        torch.cuda.synchronize()
+        if reflect:  # |c|, then 2 (n - 1) - c past the end, then clamped
+            i = np.abs(c)
+            i = np.clip(np.where(i >= n, 2 * (n - 1) - i, i), 0, n - 1)
+            ref = x[:, i]
+        else:
+            two = {F32: np.float32(2.0), BF16: np.uint16(0x4000), I64: np.int64(2)}[dt]
+            ref = np.where((c >= 0) & (c < n), x[:, np.clip(c, 0, n - 1)], two)
+        assert_bitexact(to_host(out, dt), np.ascontiguousarray(ref.astype(x.dtype)), f"pad reflect={reflect}")
+
+
 # (rows before the concat dim, source extents, elements after it, dtype, first-element offset of
 # the sources and the output): one column block, several, a row of columns just past one, more
 # sources than one launch holds, empty sources, every vector width, one row and many
