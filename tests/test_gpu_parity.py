@@ -414,6 +414,21 @@ def test_bias_act(orc, dev, act, xdt, odt):
     assert_close(to_host(y, odt), orc.bias_act(xo, xdt, None, F32, odt, act), odt, "tail")
 
 
+# an f32 bias beside 2-byte operands: columns that are whole 8-element groups, multiples of 4
+# only, and neither (the element kernel); fewer groups than a block has threads, and a ragged last block
+@pytest.mark.parametrize("rows,cols", [(1, 8), (3, 4), (7, 12), (513, 16), (65, 260), (33, 1536), (9, 30)])
+@pytest.mark.parametrize("dt", [BF16, F16])
+def test_bias_act_f32_bias_widths(orc, dev, rows, cols, dt):
+    say(f"bias_act f32 bias rows={rows} cols={cols} dt={dt}")
+    x = inp(orc, (rows, cols), 24, rows, dt, std=2.0)
+    b = inp(orc, (cols,), 25, cols)
+    for act in (1, 2, 3):
+        y = empty((rows, cols), dt)
+        mbrt.bias_act(to_dev(x, dt), to_dev(b, F32), y, act)
+        torch.cuda.synchronize()
+        assert_close(to_host(y, dt), orc.bias_act(x, dt, b, F32, dt, act), dt, f"act {act}")
+
+
 def test_glu_bl2b_full(orc, dev):
     say("BL-2b GLU bf16 [48060,3072]")
     x = inp(orc, (48060, 3072), SEED[2], 2, BF16, std=1.5)
