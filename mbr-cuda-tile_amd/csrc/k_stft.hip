@@ -6,27 +6,31 @@
 // with the standard real-input split X[f] = (Z[f] + Z*[1024-f])/2 - i W^f (Z[f] -
 // Z*[1024-f])/2 (W = exp(-2 pi i / 2048)), and the inverse split for the iSTFT.
 // One wave transforms one frame; lane l holds z[l + 64a], a = 0..15, in registers.  The
-// 1024-point FFT runs as three Stockham passes, radix 16 (in registers), 16 and 4, with
-// two exchanges through the frame's LDS slot (index p stored at p + p/16, which keeps
-// both the strided and the contiguous access patterns free of bank conflicts).  The STFT
-// takes the last pass's butterflies in mirror pairs so the real split needs no exchange.
+// 1024-point FFT runs as three Stockham passes, radix 16, 16 and 4, with two exchanges
+// through the frame's LDS slot, real parts and then imaginary parts (fft1024).  The last
+// pass takes its butterflies in mirror pairs, so the real split needs no exchange.
 //
-// Workgroup = kTF waves = kTF consecutive frames of one signal.  The frames' spectra stay
-// in LDS so that the [B, F, T] layout is written (STFT) or read (iSTFT) as runs of kTF
+// Workgroup = kTF waves = kTF consecutive frames of one signal.  The frames' spectra pass
+// through LDS so that the [B, F, T] layout is written (STFT) or read (iSTFT) as runs of kTF
 // consecutive frames per bin, instead of one 8-byte element per 8*T bytes.
 //
 // STFT   one kernel: the workgroup's sample span ((kTF - 1) hop + 2048 samples, reflect
 //        padded at the signal ends) and the window are staged once into the frame slots
-//        with coalesced loads (for hops up to 1910; larger hops read frame by frame), each
-//        wave takes its windowed frame from there, then FFT, real split, optional
-//        1/sqrt(2048), transposed store.
+//        with coalesced loads (hops up to 658; the span alone up to 950; larger hops read
+//        frame by frame), each wave takes its windowed frame from there, then FFT, real
+//        split, transposed store.  The split's 1/2 and the optional 1/sqrt(2048) scale the
+//        window.
 // iSTFT  two kernels: (1) per block of kTF frames of one signal: transposed spectrum load
-//        (f32 or bf16, times sqrt(2048) when normalized), inverse split, inverse FFT,
-//        window and 1/2048 into the frame's LDS slot, then the block's frames overlap-added
-//        in LDS (frame order) into a partial signal in a caller workspace; (2) per output
-//        sample: the partials of the blocks covering it (block order), divided by the
-//        window sum of squares where that exceeds 1e-8; centre trim and the `length` trim /
-//        zero fill are part of the same pass.  No atomics: the result is deterministic.
+//        (f32 or bf16), inverse split, inverse FFT, window, then the block's frames
+//        overlap-added in LDS (frame order) into a partial signal in a caller workspace;
+//        (2) per output sample: the partials of the blocks covering it (block order), times
+//        1/2048 (sqrt(2048)/2048 when normalized), divided by the window sum of squares where
+//        that exceeds 1e-8; centre trim and the `length` trim / zero fill are part of the
+//        same pass.  No atomics: the result is deterministic.
+//
+// LDS costs that the layouts below are chosen for (measured, cycles per wave instruction
+// without conflicts): 32-bit reads and writes 2 (32 lanes a cycle on 32 banks), 64-bit reads 2
+// (32 lanes on 64 banks), 64-bit writes 4 (16 lanes on 32 banks), 128-bit reads 4, writes 8.
 #include "abi_common.hpp"
 
 #include <atomic>
@@ -38,38 +42,37 @@ namespace {
 
 constexpr int kN = 2048;        // n_fft = win_length
 constexpr int kBins = kN / 2 + 1;
-#ifndef MBRT_STFT_TF
-#define MBRT_STFT_TF 8
+constexpr int kTF = 8;          // frames per workgroup, one wave per frame
+constexpr int kNT = 64 * kTF;   // threads per workgroup
+#ifndef MBRT_STFT_SUB
+#define MBRT_STFT_SUB 4
 #endif
-// Frames per workgroup; one wave per frame.  A workgroup holds kTF frame slots and the
-// twiddle table in LDS (78 KB at kTF = 8: two workgroups, 16 waves, per CU).
-constexpr int kTF = MBRT_STFT_TF;
+constexpr int kSub = MBRT_STFT_SUB;         // frames of an STFT workgroup that takes part of a group
 #ifndef MBRT_STFT_XCD
 #define MBRT_STFT_XCD 32
 #endif
 #ifndef MBRT_ISTFT_XCD
 #define MBRT_ISTFT_XCD 8
 #endif
+#ifndef MBRT_STFT_WPE
+#define MBRT_STFT_WPE 4
+#endif
+#ifndef MBRT_ISTFT_WPE
+#define MBRT_ISTFT_WPE 4
+#endif
+// MBRT_STFT_WPE, MBRT_ISTFT_WPE: waves per SIMD the register budgets allow for at least.  The STFT
+// needs 70 VGPRs (three workgroups, 24 waves, per CU by registers).  Held to 64 for four, it
+// spills 28 bytes a lane: 21.7 us against 21.4 on the chunk.
+//
 // Frame blocks are dealt to the XCDs in runs of this many consecutive blocks, so the blocks
 // that share the cache lines of a bin row ([B, 1025, T] holds kTF frames of a bin in
-// 8 kTF bytes) meet in one L2, and so do the STFT's overlapping sample spans.  Measured on
-// the chunk (8 signals, 801 blocks): STFT 31.2-31.5 us with runs of 8, 30.6-30.8 with 16,
-// 29.7-30.1 with 32 (kept), 34.2 with 64; the iSTFT block kernel moved by under 1 % and
-// keeps 8.
+// 8 kTF bytes) meet in one L2, and so do the STFT's overlapping sample spans.
 constexpr uint32_t kXcdRun = MBRT_STFT_XCD;
 constexpr uint32_t kXcdRunInv = MBRT_ISTFT_XCD;
-// LDS slot of one frame, in complex elements: holds padded indices up to pad(1024) = 1088;
-// 1092 complex = 2184 words = 8 (mod 64) words, so the transposed pass (kTF lanes of one
-// bin reading kTF slots) spreads over all banks.
-constexpr int kSlot = 1092;
-constexpr int kTwHalf = 1024;  // LDS twiddles W^i, i < 1024 (W^(i + 1024) = -W^i)
-// W^i sits at i + i/32 in LDS: the strided index sets of the passes (8qk over k, 2q(l + 64s)
-// over l) then fall on distinct banks.
-constexpr int kTwSlots = kTwHalf + kTwHalf / 32;
-__device__ __forceinline__ int tw_pos(int i) { return i + (i >> 5); }
-static_assert(kTF == 4 || kTF == 8 || kTF == 16, "frames per workgroup");
-
-__device__ __forceinline__ int pad16(int p) { return p + (p >> 4); }
+// LDS slot of one frame, in floats: one component (real, then imaginary) of 1024 points at
+// padded indices (up to 1071), or half a spectrum (513 complex, and two more places) on its
+// way out.  Eight of them and the twiddles are 38.8 KB.
+constexpr int kSlot = 1088;
 
 // ---- twiddles W^i = exp(-2 pi i i / 2048), built at compile time -----------------------
 // cos/sin on [0, pi/4] by their Taylor series in double, extended to the circle by the
@@ -115,7 +118,35 @@ constexpr TwiddleTable make_twiddles() {
     return t;
 }
 
-__constant__ const TwiddleTable kTwiddles = make_twiddles();
+// The twiddles a workgroup keeps in LDS, each read at a lane-linear address plus a constant
+// (no index arithmetic, no bank conflicts), forward values:
+//   V  W256^(q n),  q = 1..3, n = k + 16 r < 64   pass 2, between its two radix-4 steps
+//   U  W64^(q k),   q = 1..3, k < 16              pass 2, on its inputs
+//   P  W1024^(q l), q = 1..3, l <= 64             pass 3 (further ones by reflection)
+//   S  W2048^l,     l <= 64                       real split (further ones by rotation)
+constexpr int kTwV = 0, kTwU = kTwV + 3 * 64, kTwP = kTwU + 3 * 16, kTwS = kTwP + 3 * 65, kTwSlots = kTwS + 65;
+static_assert(kTwSlots <= kNT, "one twiddle per thread");
+
+struct FftTable {
+    float v[2 * kTwSlots];
+};
+constexpr FftTable make_fft_table() {
+    const TwiddleTable w = make_twiddles();
+    FftTable t{};
+    auto put = [&](int at, int i) {
+        t.v[2 * at] = w.v[2 * i];
+        t.v[2 * at + 1] = w.v[2 * i + 1];
+    };
+    for (int q = 1; q <= 3; ++q) {
+        for (int n = 0; n < 64; ++n) put(kTwV + (q - 1) * 64 + n, 8 * q * n);
+        for (int k = 0; k < 16; ++k) put(kTwU + (q - 1) * 16 + k, 32 * q * k);
+        for (int l = 0; l <= 64; ++l) put(kTwP + (q - 1) * 65 + l, 2 * q * l);
+    }
+    for (int l = 0; l <= 64; ++l) put(kTwS + l, l);
+    return t;
+}
+
+__constant__ const FftTable kFftTable = make_fft_table();
 
 struct cf {
     float x, y;
@@ -128,28 +159,13 @@ template <bool INV>
 __device__ __forceinline__ cf rot(cf a) {
     return INV ? cf{-a.y, a.x} : cf{a.y, -a.x};
 }
-// W^i (forward) or its conjugate (inverse), 0 <= i < 2048, from the LDS half table:
-// W^(i + 1024) = -W^i flips both signs.
+// a w (forward) or a conj(w) (inverse)
 template <bool INV>
-__device__ __forceinline__ cf twiddle(const float2* tw, int i) {
-    const float2 t = tw[tw_pos(i & (kTwHalf - 1))];
-    const uint32_t s = (uint32_t)(i >> 10) << 31;
-    return {__uint_as_float(__float_as_uint(t.x) ^ s),
-            __uint_as_float(__float_as_uint(t.y) ^ s ^ (INV ? 0x80000000u : 0u))};
+__device__ __forceinline__ cf cmulw(cf a, cf w) {
+    return INV ? cf{a.x * w.x + a.y * w.y, a.y * w.x - a.x * w.y} : cmul(a, w);
 }
-
-// Copies W^i, i < 1024, into the workgroup's LDS table (all threads take part).
-template <int NT>
-__device__ __forceinline__ void load_twiddles(float2* tw) {
-    static_assert(kTwHalf % NT == 0, "threads per workgroup divide the table");
-    constexpr int kPer = kTwHalf / NT;
-    const float2* src = reinterpret_cast<const float2*>(kTwiddles.v);
-    float2 t[kPer];  // every load in flight before the first LDS write
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) t[k] = src[threadIdx.x + k * NT];
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) tw[tw_pos(threadIdx.x + k * NT)] = t[k];
-}
+// exp(-i angle) from the angle's cosine and sine
+__device__ __forceinline__ cf unit(float c, float s) { return {c, -s}; }
 
 template <bool INV>
 __device__ __forceinline__ void dft4(cf& a0, cf& a1, cf& a2, cf& a3) {
@@ -170,7 +186,25 @@ __device__ __forceinline__ cf mul_w16(cf a) {
     return cmul(a, cf{re, INV ? -im : im});
 }
 
-// 16-point DFT in place: v[r] <- sum_q v[q] W16^(q r)  (radix 4 x 4)
+// Second half of a 16-point DFT (radix 4 x 4): v[q0 + 4 r0] holds the twiddled outputs of the
+// first radix-4 step; v[r0 + 4 r1] <- their DFT over q0.
+template <bool INV>
+__device__ __forceinline__ void dft16_tail(cf (&v)[16]) {
+    cf o[16];
+#pragma unroll
+    for (int r0 = 0; r0 < 4; ++r0) {
+        cf a0 = v[4 * r0], a1 = v[4 * r0 + 1], a2 = v[4 * r0 + 2], a3 = v[4 * r0 + 3];
+        dft4<INV>(a0, a1, a2, a3);
+        o[r0] = a0;
+        o[r0 + 4] = a1;
+        o[r0 + 8] = a2;
+        o[r0 + 12] = a3;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = o[r];
+}
+
+// 16-point DFT in place: v[r] <- sum_q v[q] W16^(q r)
 template <bool INV>
 __device__ __forceinline__ void dft16(cf (&v)[16]) {
 #pragma unroll
@@ -185,19 +219,7 @@ __device__ __forceinline__ void dft16(cf (&v)[16]) {
     v[7] = mul_w16<INV, 3>(v[7]);
     v[11] = mul_w16<INV, 6>(v[11]);
     v[15] = mul_w16<INV, 9>(v[15]);
-    // DFT over q0 for each r0: inputs v[4 r0 + q0], outputs V[r0 + 4 r1]
-    cf o[16];
-#pragma unroll
-    for (int r0 = 0; r0 < 4; ++r0) {
-        cf a0 = v[4 * r0], a1 = v[4 * r0 + 1], a2 = v[4 * r0 + 2], a3 = v[4 * r0 + 3];
-        dft4<INV>(a0, a1, a2, a3);
-        o[r0] = a0;
-        o[r0 + 4] = a1;
-        o[r0 + 8] = a2;
-        o[r0 + 12] = a3;
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = o[r];
+    dft16_tail<INV>(v);
 }
 
 // Orders this wave's LDS accesses: lanes of one wave exchange data through the slot.
@@ -213,74 +235,116 @@ __device__ __forceinline__ cf lds_ld(const float2* s, int i) {
 }
 __device__ __forceinline__ void lds_st(float2* s, int i, cf v) { s[i] = make_float2(v.x, v.y); }
 
-// Passes 1 and 2 of the 1024-point FFT of one frame by one wave.  In: lane l holds z[l + 64a]
-// in v[a].  Out: the slot holds y2 (pass-2 output) at padded indices.  Previous slot
-// contents are overwritten.
+// One exchange of the FFT: element r of a lane's v goes to slot index at(r), element q of the
+// result comes from from(q).  The slot holds one component at a time, half the LDS of a
+// complex exchange, at a third more LDS cycles (2 + 2 per component against 4 + 2).
+template <class At, class From>
+__device__ __forceinline__ void exchange(cf (&v)[16], float* slot, At at, From from) {
+    float re[16];
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) slot[at(r)] = v[r].x;
+    wave_lds_sync();
+#pragma unroll
+    for (int q = 0; q < 16; ++q) re[q] = slot[from(q)];
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) slot[at(r)] = v[r].y;
+    wave_lds_sync();
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = cf{re[q], slot[from(q)]};
+}
+
+// 1024-point FFT of one frame by one wave.  In: lane l holds z[l + 64a] in v[a].  Out: the four
+// radix-4 butterflies of the last pass that the lane took, in mirror pairs: butterfly j yields
+// Z[j + 256 r], r = 0..3, in its z[r], for
+//   A: j = l,   B: j = 256 - l (lane 0: 128),   C: j = 128 + m,   D: j = 128 - m
+// with m = l (lane 0: 64), so that Z[f] and Z[1024 - f] of every f sit in one lane.
 template <bool INV>
-__device__ __forceinline__ void fft_pass12(cf (&v)[16], float2* slot, const float2* tw, int lane) {
+__device__ __forceinline__ void fft1024(cf (&v)[16], float* slot, const float2* tw, int lane, cf (&zA)[4], cf (&zB)[4],
+                                        cf (&zC)[4], cf (&zD)[4]) {
+    const int k = lane & 15;
     // pass 1: radix 16 over z[j + 64q]; y[16j + r]
     dft16<INV>(v);
-    wave_lds_sync();
+    // (index i at i + i / 32: 32 lanes 16 apart and 32 consecutive ones both cover the 32 banks)
+    const int w1 = 16 * lane + (lane >> 1), r1 = lane + (lane >> 5);
+    exchange(v, slot, [&](int r) { return w1 + r; }, [&](int q) { return r1 + 66 * q; });
+    // pass 2: radix 16, span 16: inputs y[j + 64q] W256^(qk), k = j % 16; outputs
+    // y2[(j - k) 16 + k + 16 r].  With q = q0 + 4 q1, W256^(qk) = W64^(q1 k) W256^(q0 k): the first
+    // factor goes on the inputs, the second joins the W16^(q0 r0) between the radix-4 steps.
+    {
+        const float2* t = tw + k;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) lds_st(slot, 17 * lane + r, v[r]);
-    wave_lds_sync();
-    // pass 2: radix 16, span 16: inputs y[j + 64q] * W256^(qk), k = j % 16;
-    // outputs y2[(j - k) 16 + k + 16 r].  W^(8qk) = W^(8 q0 k) W^(32 q1 k) for q = q0 + 4 q1:
-    // six table reads and nine products instead of fifteen reads.
-    const int k = lane & 15, rb = pad16(lane);
+        for (int q1 = 1; q1 < 4; ++q1) {
+            const cf w = lds_ld(t, kTwU + (q1 - 1) * 16);
 #pragma unroll
-    for (int q = 0; q < 16; ++q) v[q] = lds_ld(slot, rb + 68 * q);
-    const cf t1 = twiddle<INV>(tw, 8 * k), t2 = twiddle<INV>(tw, 16 * k), t3 = twiddle<INV>(tw, 24 * k);
-    const cf u1 = twiddle<INV>(tw, 32 * k), u2 = twiddle<INV>(tw, 64 * k), u3 = twiddle<INV>(tw, 96 * k);
-    const cf tq0[4] = {cf{1.f, 0.f}, t1, t2, t3}, tq1[4] = {cf{1.f, 0.f}, u1, u2, u3};
+            for (int q0 = 0; q0 < 4; ++q0) v[q0 + 4 * q1] = cmulw<INV>(v[q0 + 4 * q1], w);
+        }
 #pragma unroll
-    for (int q = 1; q < 16; ++q) {
-        const int q0 = q & 3, q1 = q >> 2;
-        const cf w = q0 == 0 ? tq1[q1] : (q1 == 0 ? tq0[q0] : cmul(tq0[q0], tq1[q1]));
-        v[q] = cmul(v[q], w);
+        for (int q0 = 0; q0 < 4; ++q0) dft4<INV>(v[q0], v[q0 + 4], v[q0 + 8], v[q0 + 12]);
+#pragma unroll
+        for (int q0 = 1; q0 < 4; ++q0)
+#pragma unroll
+            for (int r0 = 0; r0 < 4; ++r0)
+                v[q0 + 4 * r0] = cmulw<INV>(v[q0 + 4 * r0], lds_ld(t, kTwV + (q0 - 1) * 64 + 16 * r0));
+        dft16_tail<INV>(v);
     }
-    dft16<INV>(v);
-    wave_lds_sync();
-    const int wb = 272 * (lane >> 4) + k;
+    const int m = lane ? lane : 64;
+    const int jb[4] = {lane, lane ? 256 - lane : 128, 128 + m, 128 - m};
+    // (index i at i + 16 (i / 256): the writes of 32 lanes are two runs of 16, 16 banks apart)
+    const int w2 = 272 * (lane >> 4) + k;
+    exchange(v, slot, [&](int r) { return w2 + 16 * r; }, [&](int q) { return jb[q >> 2] + 272 * (q & 3); });
+    // pass 3: radix 4, span 256: inputs y2[j + 256q] W1024^(qj)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) lds_st(slot, wb + 17 * r, v[r]);
-    wave_lds_sync();
-}
-
-// Radix-4 butterfly jj of pass 3 (span 256): inputs y2[jj + 256q] * W1024^(q jj) from the slot,
-// outputs Z[jj + 256 r] in z[r].
-template <bool INV>
-__device__ __forceinline__ void pass3_butterfly(const float2* slot, const float2* tw, int jj, cf (&z)[4]) {
-    const int base = jj + (jj >> 4);  // pad16(jj + 256 q) = base + 272 q
-#pragma unroll
-    for (int q = 0; q < 4; ++q) z[q] = lds_ld(slot, base + 272 * q);
-    z[1] = cmul(z[1], twiddle<INV>(tw, 2 * jj));
-    z[2] = cmul(z[2], twiddle<INV>(tw, 4 * jj));
-    z[3] = cmul(z[3], twiddle<INV>(tw, 6 * jj));
-    dft4<INV>(z[0], z[1], z[2], z[3]);
-}
-
-// 1024-point FFT of one frame by one wave.  In: lane l holds z[l + 64a] in v[a].  Out: lane
-// l holds Z[l + 64a] in v[a].
-template <bool INV>
-__device__ __forceinline__ void fft1024(cf (&v)[16], float2* slot, const float2* tw, int lane) {
-    fft_pass12<INV>(v, slot, tw, lane);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        cf z[4];
-        pass3_butterfly<INV>(slot, tw, lane + 64 * s, z);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[s + 4 * r] = z[r];
+    for (int q = 0; q < 4; ++q) {
+        zA[q] = v[q];
+        zB[q] = v[4 + q];
+        zC[q] = v[8 + q];
+        zD[q] = v[12 + q];
     }
+    constexpr float H = 0.70710678118654752440f;
+    {
+        const cf a1 = lds_ld(tw, kTwP + lane), a2 = lds_ld(tw, kTwP + 65 + lane), a3 = lds_ld(tw, kTwP + 130 + lane);
+        zA[1] = cmulw<INV>(zA[1], a1);
+        zA[2] = cmulw<INV>(zA[2], a2);
+        zA[3] = cmulw<INV>(zA[3], a3);
+        // angles q (256 - l) 2 pi / 1024 = q pi / 2 - (those of A); lane 0: q pi / 4
+        cf b1 = unit(-a1.y, a1.x), b2 = unit(-a2.x, -a2.y), b3 = unit(a3.y, -a3.x);
+        if (lane == 0) {
+            b1 = unit(H, H);
+            b2 = unit(0.0f, 1.0f);
+            b3 = unit(-H, H);
+        }
+        zB[1] = cmulw<INV>(zB[1], b1);
+        zB[2] = cmulw<INV>(zB[2], b2);
+        zB[3] = cmulw<INV>(zB[3], b3);
+    }
+    {
+        // angles q (128 +- m) 2 pi / 1024 = q pi / 4 +- phi_q
+        const cf p1 = lds_ld(tw, kTwP + m), p2 = lds_ld(tw, kTwP + 65 + m), p3 = lds_ld(tw, kTwP + 130 + m);
+        const float s1 = H * (p1.x - p1.y), d1 = H * (p1.x + p1.y);  // h (cos + sin), h (cos - sin)
+        const float s3 = H * (p3.x - p3.y), d3 = H * (p3.x + p3.y);
+        zC[1] = cmulw<INV>(zC[1], unit(d1, s1));
+        zD[1] = cmulw<INV>(zD[1], unit(s1, d1));
+        zC[2] = cmulw<INV>(zC[2], unit(p2.y, p2.x));
+        zD[2] = cmulw<INV>(zD[2], unit(-p2.y, p2.x));
+        zC[3] = cmulw<INV>(zC[3], unit(-s3, d3));
+        zD[3] = cmulw<INV>(zD[3], unit(-d3, s3));
+    }
+    dft4<INV>(zA[0], zA[1], zA[2], zA[3]);
+    dft4<INV>(zB[0], zB[1], zB[2], zB[3]);
+    dft4<INV>(zC[0], zC[1], zC[2], zC[3]);
+    dft4<INV>(zD[0], zD[1], zD[2], zD[3]);
 }
 
-// Real-input split of one mirror pair: from Z[f] and Z[1024 - f] (W^f = wf) writes X[f] and
-// X[1024 - f] into the slot.  f = 0 (with zg = Z[0]) yields X[0] and X[1024].
-__device__ __forceinline__ void r2c_pair(float2* slot, int f, cf zf, cf zg, cf wf) {
+// Real-input split of one mirror pair: X[f] and X[1024 - f], twice over, from Z[f] and
+// Z[1024 - f] (W^f = wf); f = 0 with zg = Z[0] yields X[0] and X[1024].  (The factor 1/2 is
+// folded into the window.)
+__device__ __forceinline__ void r2c_pair(cf zf, cf zg, cf wf, cf& xf, cf& xg) {
     const cf A{zf.x + zg.x, zf.y - zg.y}, Bv{zf.x - zg.x, zf.y + zg.y};
     const cf P = cmul(wf, Bv);
-    lds_st(slot, pad16(f), cf{0.5f * (A.x + P.y), 0.5f * (A.y - P.x)});
-    lds_st(slot, pad16(kN / 2 - f), cf{0.5f * (A.x - P.y), -0.5f * (A.y + P.x)});
+    xf = cf{A.x + P.y, A.y - P.x};
+    xg = cf{A.x - P.y, -(A.y + P.x)};
 }
 
 // ---- STFT -------------------------------------------------------------------------------
@@ -290,384 +354,441 @@ struct StftArgs {
     float2* out;       // [B, 1025, T] complex
     int L;
     uint32_t T;        // frames per signal
-    FastDiv ntb;       // workgroups per signal: block index -> (signal, block in signal)
+    FastDiv ntb;       // groups of kTF frames per signal: group -> (signal, group in signal)
+    uint32_t whole;    // groups that one workgroup takes whole
     int hop;
     int offset;        // 1024 when centred (reflect padding), else 0
-    int wvec;          // window is 8-byte aligned: read it as float2
-    int xvec;          // signal is 16-byte aligned: stage it with float4 loads
-    int staged;        // the workgroup's sample span and the window fit its frame slots
-    float norm;
+    int staged;        // the frame slots hold the workgroup's sample span (1), and the window too (2)
+    float scale;       // 1/2 (of the real split), times 1/sqrt(2048) when normalized
 };
 
-// Windowed frame of sample pairs: v[q] = (x[n] w[n], x[n+1] w[n+1]), n = 2 (lane + 64 q).
-__device__ __forceinline__ void load_frame(const StftArgs& a, uint32_t b, uint32_t t, int lane, cf (&v)[16]) {
-    const float* xb = a.x + (int64_t)b * a.L;
-    const int start = (int)t * a.hop - a.offset;
-    float2 w[16];
-    if (a.wvec) {
-#pragma unroll
-        for (int q = 0; q < 16; ++q) w[q] = reinterpret_cast<const float2*>(a.w)[lane + 64 * q];
-    } else {
-#pragma unroll
-        for (int q = 0; q < 16; ++q) w[q] = make_float2(a.w[2 * (lane + 64 * q)], a.w[2 * (lane + 64 * q) + 1]);
-    }
+// Sample c of a signal of L samples, reflected once about the ends, then clamped (the
+// reference's pad_reflect rule).
+__device__ __forceinline__ int reflect_index(int c, int L) {
+    if (c < 0) c = -c;
+    if (c >= L) c = 2 * (L - 1) - c;
+    return c < 0 ? 0 : (c > L - 1 ? L - 1 : c);
+}
+
+typedef float f32x2_any __attribute__((ext_vector_type(2), aligned(4)));  // two floats at any float address
+__device__ __forceinline__ float2 ld2_any(const float* p) {
+    const f32x2_any v = *reinterpret_cast<const f32x2_any*>(p);
+    return make_float2(v.x, v.y);
+}
+
+// Samples n = 2 (lane + 64 q), n + 1 of a frame that starts at sample `start` of signal xb, straight
+// from memory.
+__device__ __forceinline__ void load_frame(const StftArgs& a, const float* xb, int start, int lane, cf (&v)[16]) {
     if (start >= 0 && start + kN <= a.L) {
-        const float* xs = xb + start;
-        if ((reinterpret_cast<uintptr_t>(xs) & 7) == 0) {
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const float2 p = reinterpret_cast<const float2*>(xs)[lane + 64 * q];
-                v[q] = cf{p.x * w[q].x, p.y * w[q].y};
-            }
-        } else {
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int n = 2 * (lane + 64 * q);
-                v[q] = cf{xs[n] * w[q].x, xs[n + 1] * w[q].y};
-            }
-        }
-    } else {
-        // reflect once about the ends, then clamp (the reference's pad_reflect rule)
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
-            const int n = 2 * (lane + 64 * q);
-            float e[2];
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                int c = start + n + h;
-                if (c < 0) c = -c;
-                if (c >= a.L) c = 2 * (a.L - 1) - c;
-                c = c < 0 ? 0 : (c > a.L - 1 ? a.L - 1 : c);
-                e[h] = xb[c];
-            }
-            v[q] = cf{e[0] * w[q].x, e[1] * w[q].y};
+            const float2 p = ld2_any(xb + start + 2 * (lane + 64 * q));
+            v[q] = cf{p.x, p.y};
         }
-    }
-}
-
-// Stages the workgroup's window (2048 floats) and sample span ((nf - 1) hop + 2048 floats
-// from sample s of signal b) into LDS: the span with aligned float4 loads when it lies
-// inside the signal, else sample by sample through the reflect-then-clamp rule.  Returns
-// the span's offset in the staging area.
-template <int NT>
-__device__ __forceinline__ int stage_span(const StftArgs& a, float* stage, uint32_t b, int s, int span) {
-    // Loads are issued in groups of 4 per thread before their LDS writes, so that each
-    // thread has several in flight.
-    const int tid = threadIdx.x;
-    if (a.wvec) {
-        static_assert((kN / 2) % NT == 0, "threads per workgroup divide the window");
-        constexpr int kPer = kN / 2 / NT;
-        float2 wv[kPer];
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) wv[k] = reinterpret_cast<const float2*>(a.w)[tid + k * NT];
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) reinterpret_cast<float2*>(stage)[tid + k * NT] = wv[k];
     } else {
-        constexpr int kPer = kN / NT;
-        float wv[kPer];
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) wv[k] = a.w[tid + k * NT];
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) stage[tid + k * NT] = wv[k];
-    }
-    float* xst = stage + kN;
-    if (a.xvec && s >= 0 && s + span <= a.L) {
-        const int64_t base = (int64_t)b * a.L + s, end = base + span;
-        const int64_t a4 = base & ~int64_t(3);  // >= 0; float4 loads from a4 are 16-byte aligned
-        const int xoff = (int)(base - a4), n4 = (xoff + span + 3) >> 2;
-        for (int i0 = tid; i0 < n4; i0 += 4 * NT) {
-            float4 v[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int i = i0 + k * NT;
-                const int64_t e = a4 + 4 * (int64_t)i;
-                if (i >= n4) {
-                    v[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                } else if (e + 4 <= end) {
-                    v[k] = *reinterpret_cast<const float4*>(a.x + e);
-                } else {  // the last partial vector: nothing at or past the span's end is read
-                    v[k].x = e < end ? a.x[e] : 0.0f;
-                    v[k].y = e + 1 < end ? a.x[e + 1] : 0.0f;
-                    v[k].z = e + 2 < end ? a.x[e + 2] : 0.0f;
-                    v[k].w = 0.0f;
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (i0 + k * NT < n4) reinterpret_cast<float4*>(xst)[i0 + k * NT] = v[k];
+        for (int q = 0; q < 16; ++q) {
+            const int n = start + 2 * (lane + 64 * q);
+            v[q] = cf{xb[reflect_index(n, a.L)], xb[reflect_index(n + 1, a.L)]};
         }
-        return xoff;
     }
-    const float* xb = a.x + (int64_t)b * a.L;
-    for (int j0 = tid; j0 < span; j0 += 4 * NT) {
-        float v[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            // reflect once about the ends, then clamp (the reference's pad_reflect rule)
-            int c = s + j0 + k * NT;
-            if (c < 0) c = -c;
-            if (c >= a.L) c = 2 * (a.L - 1) - c;
-            c = c < 0 ? 0 : (c > a.L - 1 ? a.L - 1 : c);
-            v[k] = j0 + k * NT < span ? xb[c] : 0.0f;
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (j0 + k * NT < span) xst[j0 + k * NT] = v[k];
-    }
-    return 0;
 }
 
-// The staged prologue when the workgroup's span lies inside its signal and the window and
-// signal are aligned (the common case): the window, the twiddles and the span (KS float4
-// per thread, indices clamped to the span's last whole vector) are all loaded before the
-// first LDS write, so the workgroup pays one memory round trip instead of one per load
-// group.  The span's last partial vector (1..3 samples) is read by thread 0.  Returns the
-// span's offset in the staging area, as stage_span.
-template <int NT, int KS>
-__device__ __forceinline__ int stage_all(const StftArgs& a, float* stage, float2* tw, uint32_t b, int s, int span) {
+__device__ __forceinline__ float4 ld4_any(const float* p) { return __builtin_bit_cast(float4, ld_any<0, 4>(p)); }
+
+// Stages `span` (>= 2048) samples from sample s of signal xb into LDS, the even ones at xst and the
+// odd ones KH floats further (a frame's sample pairs are then two runs of consecutive words
+// whatever the frame's first sample), and the twiddles and (WIN) the scaled window beside
+// them.  Every load is in flight before the first LDS write where the span lies inside the
+// signal: KS vectors per thread, the vector index clamped to the last whole one.
+template <int KS, int KH, bool WIN>
+__device__ __forceinline__ void stage_span(const StftArgs& a, float* xst, float* wst, float2* tw, const float* xb, int s,
+                                           int span) {
     const int tid = threadIdx.x;
-    const int64_t base = (int64_t)b * a.L + s, end = base + span;
-    const int64_t a4 = base & ~int64_t(3);
-    const int xoff = (int)(base - a4), n4 = (xoff + span + 3) >> 2;
-    const int nfull = (int)((end - a4) >> 2);  // vectors wholly inside the span (>= 1)
-    constexpr int kW = kN / 2 / NT, kT = kTwHalf / NT;
-    float2 wv[kW], tv[kT];
-    float4 xv[KS];
-    const float2* tsrc = reinterpret_cast<const float2*>(kTwiddles.v);
+    const float2 t = reinterpret_cast<const float2*>(kFftTable.v)[min(tid, kTwSlots - 1)];
+    float4 w = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if constexpr (WIN) w = ld4_any(a.w + 4 * tid);
+    if (s >= 0 && s + span <= a.L) {
+        const int last = (span >> 2) - 1, tail = min((span & ~3) + tid, span - 1);
+        float4 xv[KS];
 #pragma unroll
-    for (int k = 0; k < kW; ++k) wv[k] = reinterpret_cast<const float2*>(a.w)[tid + k * NT];
+        for (int k = 0; k < KS; ++k) xv[k] = ld4_any(xb + s + 4 * min(tid + kNT * k, last));
+        float xt = 0.0f;
+        if (tid < 3) xt = xb[s + tail];
 #pragma unroll
-    for (int k = 0; k < kT; ++k) tv[k] = tsrc[tid + k * NT];
-    const float4* x4 = reinterpret_cast<const float4*>(a.x + a4);
+        for (int k = 0; k < KS; ++k) {
+            const int i = 2 * min(tid + kNT * k, last);
+            *reinterpret_cast<float2*>(xst + i) = make_float2(xv[k].x, xv[k].z);
+            *reinterpret_cast<float2*>(xst + KH + i) = make_float2(xv[k].y, xv[k].w);
+        }
+        if (tid < 3) xst[(tail & 1) * KH + (tail >> 1)] = xt;
+    } else {
+        for (int j0 = tid; j0 < span; j0 += 6 * kNT) {
+            float xv[6];
 #pragma unroll
-    for (int k = 0; k < KS; ++k) xv[k] = x4[min(tid + k * NT, nfull - 1)];
-    float tail[3] = {0.0f, 0.0f, 0.0f};
-    if (tid == 0 && n4 > nfull) {
+            for (int k = 0; k < 6; ++k) xv[k] = xb[reflect_index(s + min(j0 + k * kNT, span - 1), a.L)];
 #pragma unroll
-        for (int e = 0; e < 3; ++e) {
-            const int64_t q = a4 + 4 * (int64_t)nfull + e;
-            tail[e] = q < end ? a.x[q] : 0.0f;
+            for (int k = 0; k < 6; ++k) {
+                const int i = j0 + k * kNT;
+                if (i < span) xst[(i & 1) * KH + (i >> 1)] = xv[k];
+            }
         }
     }
-#pragma unroll
-    for (int k = 0; k < kW; ++k) reinterpret_cast<float2*>(stage)[tid + k * NT] = wv[k];
-#pragma unroll
-    for (int k = 0; k < kT; ++k) tw[tw_pos(tid + k * NT)] = tv[k];
-    float* xst = stage + kN;
-    // unconditional writes (threads past the span rewrite its last whole vector with the
-    // same bytes): a predicated write would let the compiler sink each load into its branch
-    // and wait for it there, one round trip per load
-#pragma unroll
-    for (int k = 0; k < KS; ++k) reinterpret_cast<float4*>(xst)[min(tid + k * NT, nfull - 1)] = xv[k];
-    if (tid == 0 && n4 > nfull) {
-#pragma unroll
-        for (int e = 0; e < 3; ++e) xst[4 * nfull + e] = tail[e];
-    }
-    return xoff;
+    if (tid < kTwSlots) tw[tid] = t;
+    if constexpr (WIN)
+        *reinterpret_cast<float4*>(wst + 4 * tid) = make_float4(w.x * a.scale, w.y * a.scale, w.z * a.scale, w.w * a.scale);
 }
 
-template <int TF>
-__global__ __launch_bounds__(64 * TF) void stft_kernel(StftArgs a) {
-    constexpr int NT = 64 * TF;
-    __shared__ __attribute__((aligned(16))) float2 lds[TF * kSlot + kTwSlots];
-    float2* tw = lds + TF * kSlot;
+// Bound by vector arithmetic and LDS together, and by how evenly the CUs are loaded.  Per frame:
+// 826 vector instructions (8.6 us of SIMD time on the chunk, [8, 352800] -> 6,408 frames) and 685
+// LDS cycles (7.1 us), beside 64 MB of HBM (11 us).  The kernel that kept whole complex slots (two
+// workgroups per CU) and computed its twiddle indices took 1,111 and 720 cycles, of which 153 were bank
+// conflicts: 25.5 us.  Half slots, per-lane twiddle tables and layouts without conflicts: 21.4.
+// The same with layouts padded by p/16, whose 32-bit reads conflict: 28.4.
+__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(MBRT_STFT_WPE))) void stft_kernel(StftArgs a) {
+    __shared__ __attribute__((aligned(16))) float lds[kTF * kSlot + 2 * kTwSlots];
+    float2* tw = reinterpret_cast<float2*>(lds + kTF * kSlot);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    // workgroup = frames t0 .. t0 + nf - 1 of signal b
-    uint32_t b, tb;
-    fdivmod(xcd_runs<kXcdRun>(blockIdx.x, gridDim.x), a.ntb, b, tb);
-    const uint32_t t0 = tb * TF;
-    const int nf = (int)min((uint32_t)TF, a.T - t0);
+    // workgroup = frames t0 .. t0 + nf - 1 of signal b: one of the first `whole` groups of kTF frames,
+    // or a kSub-frame part of one of the others
+    uint32_t b, tb, sub = 0, nfm = kTF, g = xcd_runs<kXcdRun>(blockIdx.x, min(a.whole, gridDim.x));
+    if (blockIdx.x >= a.whole) {
+        const uint32_t q = blockIdx.x - a.whole;
+        g = a.whole + q / (kTF / kSub);
+        sub = q % (kTF / kSub) * kSub;
+        nfm = kSub;
+    }
+    fdivmod(g, a.ntb, b, tb);
+    const uint32_t t0 = tb * kTF + sub;
+    if (t0 >= a.T) return;
+    const int nf = (int)min(nfm, a.T - t0);
     const bool live = wave < nf;
+    const float* xb = a.x + (int64_t)b * a.L;
+    const int s = (int)t0 * a.hop - a.offset;
     cf v[16];
     if (a.staged) {
-        // the frames of a workgroup overlap (hop < 2048): their span and the window are read
+        // the frames of a workgroup overlap (hop < 2048): their span (and the window) are read
         // from HBM once, coalesced, into the frame slots, and each wave takes its frame there
-        const int s = (int)t0 * a.hop - a.offset;
-        float* stage = reinterpret_cast<float*>(lds);
+        constexpr int KH2 = (kTF * kSlot - kN) / 2, KH1 = kTF * kSlot / 2;
+        float* xst = lds + (a.staged == 2 ? kN : 0);
         const int span = (nf - 1) * a.hop + kN;
-        int xoff;
-        if (a.wvec && a.xvec && s >= 0 && s + span <= a.L && span + 3 <= 4 * 4 * NT) {
-            xoff = stage_all<NT, 4>(a, stage, tw, b, s, span);
-        } else {
-            xoff = stage_span<NT>(a, stage, b, s, span);
-            load_twiddles<NT>(tw);
-        }
+        if (a.staged == 2 && span <= 3 * 4 * kNT) stage_span<3, KH2, true>(a, xst, lds, tw, xb, s, span);
+        else if (a.staged == 2) stage_span<4, KH2, true>(a, xst, lds, tw, xb, s, span);
+        else stage_span<5, KH1, false>(a, xst, lds, tw, xb, s, span);
         __syncthreads();
         if (live) {
-            const float* xs = stage + kN + xoff + wave * a.hop;
+            // samples h + 2 m and h + 2 m + 1 of the span, h the frame's first
+            const int h = wave * a.hop, kh = a.staged == 2 ? KH2 : KH1;
+            const float* x0 = xst + (h & 1) * kh + (h >> 1) + lane;
+            const float* x1 = xst + (1 - (h & 1)) * kh + ((h + 1) >> 1) + lane;
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
-                const int n = 2 * (lane + 64 * q);
-                const float2 w = reinterpret_cast<const float2*>(stage)[lane + 64 * q];
-                v[q] = cf{xs[n] * w.x, xs[n + 1] * w.y};
+                float2 w;
+                if (a.staged == 2) {
+                    w = reinterpret_cast<const float2*>(lds)[lane + 64 * q];
+                } else {
+                    w = ld2_any(a.w + 2 * (lane + 64 * q));
+                    w = make_float2(w.x * a.scale, w.y * a.scale);
+                }
+                v[q] = cf{x0[64 * q] * w.x, x1[64 * q] * w.y};
             }
         }
         __syncthreads();  // the staging area becomes the frame slots
     } else {
-        if (live) load_frame(a, b, t0 + wave, lane, v);
-        load_twiddles<NT>(tw);
+        if (threadIdx.x < kTwSlots) tw[threadIdx.x] = reinterpret_cast<const float2*>(kFftTable.v)[threadIdx.x];
+        if (live) {
+            load_frame(a, xb, s + wave * a.hop, lane, v);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const float2 w = ld2_any(a.w + 2 * (lane + 64 * q));
+                v[q] = cf{v[q].x * (w.x * a.scale), v[q].y * (w.y * a.scale)};
+            }
+        }
         __syncthreads();
     }
+    // The spectra leave through LDS in two halves: bins f < 512, then their mirrors 1024 - f
+    // (with bin 512 = its own), both at position f of the frame's slot, rotated by the frame
+    // (f ^ 4 wave within 32) so that the transposed reads (8 frames x 4 bins in 32 lanes) fall on
+    // different banks.
+    float* slot = lds + wave * kSlot;
+    float2* sc = reinterpret_cast<float2*>(slot);
+    // places of a lane's pairs: f = p0, p0 + 256, p1 + 256, p1, p2, p2 + 256, p3 + 256, p3
+    const int rot = wave << 2, m = lane ? lane : 64;
+    const int p0 = lane ^ rot, p1 = (256 - lane) ^ rot, p2 = (128 + m) ^ rot, p3 = (128 - m) ^ rot;
+    cf xg[8];
     if (live) {
-        float2* slot = lds + wave * kSlot;
-        fft_pass12<false>(v, slot, tw, lane);
-        // pass 3 over butterflies chosen in mirror pairs (jj, 256 - jj), so that every lane
-        // holds both Z[f] and Z[1024 - f] of its outputs: lanes 1..63 take l, 256 - l,
-        // 128 + l, 128 - l; lane 0 takes 0, 128 (each its own mirror), 64, 192.
-        const int jA = lane, jB = lane ? 256 - lane : 128;
-        const int jC = lane ? 128 + lane : 64, jD = lane ? 128 - lane : 192;
         cf zA[4], zB[4], zC[4], zD[4];
-        pass3_butterfly<false>(slot, tw, jA, zA);
-        pass3_butterfly<false>(slot, tw, jB, zB);
-        pass3_butterfly<false>(slot, tw, jC, zC);
-        pass3_butterfly<false>(slot, tw, jD, zD);
+        fft1024<false>(v, slot, tw, lane, zA, zB, zC, zD);
         wave_lds_sync();
-        // real split: Z[1024 - (jA + 256 r)] is zB[3 - r] (lane 0: zA[(4 - r) % 4]); Z[1024 -
-        // (jC + 256 r)] is zD[3 - r]; lane 0 also splits butterfly 128 against itself.
+        // W^f of every pair from W^l and W^m: angles l, pi/4 -+ l, pi/2 - l, and pi/8, 3 pi/8 +- m
+        const cf sl = lds_ld(tw, kTwS + lane), sm = lds_ld(tw, kTwS + m);
+        constexpr float H = 0.70710678118654752440f, C1 = 0.92387953251128675613f, S1 = 0.38268343236508977173f;
+        auto pair = [&](int place, cf zf, cf zg, cf w, cf& g) {
+            cf x;
+            r2c_pair(zf, zg, w, x, g);
+            lds_st(sc, place, x);
+        };
+        if (lane == 0) {  // butterfly 128 is its own mirror
+            cf g;  // its mirrors wait in the slot's last two places
+            pair(128 ^ rot, zB[0], zB[3], unit(C1, S1), g);
+            lds_st(sc, kSlot / 2 - 1, g);
+            pair(384 ^ rot, zB[1], zB[2], unit(S1, C1), g);
+            lds_st(sc, kSlot / 2 - 2, g);
+            // and so is A: Z[256 (4 - r)]
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const cf za = lane ? zB[3 - r] : zA[(4 - r) & 3];
-            r2c_pair(slot, jA + 256 * r, zA[r], za, twiddle<false>(tw, jA + 256 * r));
-            r2c_pair(slot, jC + 256 * r, zC[r], zD[3 - r], twiddle<false>(tw, jC + 256 * r));
+            for (int r = 0; r < 4; ++r) zB[r] = zA[(r + 1) & 3];
         }
-        if (lane == 0) {
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-                r2c_pair(slot, 128 + 256 * r, zB[r], zB[3 - r], twiddle<false>(tw, 128 + 256 * r));
+        {
+            const float c = sl.x, n = -sl.y, p4 = H * (c + n), m4 = H * (c - n);
+            pair(p0, zA[0], zB[3], unit(c, n), xg[0]);
+            pair(p0 + 256, zA[1], zB[2], unit(m4, p4), xg[1]);
+            pair(p1 + 256, zB[1], zA[2], unit(n, c), xg[2]);
+            pair(p1, zB[0], zA[3], unit(p4, m4), xg[3]);
+        }
+        {
+            const float cm = sm.x, nm = -sm.y;
+            const float cp = C1 * cm - S1 * nm, sp = S1 * cm + C1 * nm;  // pi/8 + m
+            const float cq = C1 * cm + S1 * nm, sq = S1 * cm - C1 * nm;  // pi/8 - m
+            pair(p2, zC[0], zD[3], unit(cp, sp), xg[4]);
+            pair(p2 + 256, zC[1], zD[2], unit(sq, cq), xg[5]);
+            pair(p3 + 256, zD[1], zC[2], unit(sp, cp), xg[6]);
+            pair(p3, zD[0], zC[3], unit(cq, sq), xg[7]);
         }
     }
     __syncthreads();
-    // transposed store: thread -> (frame t0 + tl, bins fr, fr + 64, ...)
-    const int tl = threadIdx.x % TF, fr = threadIdx.x / TF;
+    // transposed store: thread -> (frame t0 + tl, bins fr + 64 i, then 1024 - fr - 64 i)
+    const int tl = threadIdx.x % kTF, fr = threadIdx.x / kTF;
+    const float2* src = reinterpret_cast<const float2*>(lds + tl * kSlot) + (fr ^ (tl << 2));
+    f32x2* dst = reinterpret_cast<f32x2*>(a.out) + ((int64_t)b * kBins * a.T + t0 + tl);
+    const int64_t step = (int64_t)64 * a.T;
+    float2 X[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) X[i] = src[64 * i];
+    __syncthreads();
+    if (tl < nf) {
+        f32x2* p = dst + (int64_t)fr * a.T;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) gst<MBRT_NT_STFT & 2>(p + i * step, f32x2{X[i].x, X[i].y});
+    }
+    if (live) {
+        lds_st(sc, p0, xg[0]);
+        lds_st(sc, p0 + 256, xg[1]);
+        lds_st(sc, p1 + 256, xg[2]);
+        lds_st(sc, p1, xg[3]);
+        lds_st(sc, p2, xg[4]);
+        lds_st(sc, p2 + 256, xg[5]);
+        lds_st(sc, p3 + 256, xg[6]);
+        lds_st(sc, p3, xg[7]);
+        if (lane == 0) {
+            lds_st(sc, 128 ^ rot, lds_ld(sc, kSlot / 2 - 1));
+            lds_st(sc, 384 ^ rot, lds_ld(sc, kSlot / 2 - 2));
+        }
+    }
+    __syncthreads();
     if (tl >= nf) return;
-    float2* dst = a.out + ((int64_t)b * kBins * a.T + t0 + tl);
-    const float2* src = lds + tl * kSlot;
-    const int64_t step = (int64_t)(NT / TF) * a.T;
-    dst += (int64_t)fr * a.T;
-#pragma unroll 4
-    for (int f = fr; f < kBins; f += NT / TF, dst += step) {
-        const float2 X = src[pad16(f)];
-        gst<MBRT_NT_STFT & 2>(reinterpret_cast<f32x2*>(dst), f32x2{X.x * a.norm, X.y * a.norm});
+    f32x2* p = dst + (int64_t)(kN / 2 - fr) * a.T;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) X[i] = src[64 * i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) gst<MBRT_NT_STFT & 2>(p - i * step, f32x2{X[i].x, X[i].y});
+    if (fr == 0) {
+        const float2 h = reinterpret_cast<const float2*>(lds + tl * kSlot)[512 + (tl << 2)];
+        gst<MBRT_NT_STFT & 2>(dst + (int64_t)512 * a.T, f32x2{h.x, h.y});
     }
 }
 
 // ---- iSTFT ------------------------------------------------------------------------------
 // Block kernel: one workgroup = kTF consecutive frames of one signal.  Their spectra are
-// loaded transposed, each wave inverts one frame and leaves it, windowed and scaled, in its
-// LDS slot; the workgroup then overlap-adds its frames in LDS (frame order) and writes the
-// block's partial signal, (nf - 1) hop + 2048 samples from sample t0 hop.  The final
-// kernel adds, per output sample, the partials of the blocks that cover it (block order)
-// and divides by the window sum.
+// loaded transposed, each wave inverts one frame, and the workgroup overlap-adds its frames
+// in LDS (frame order) and writes the block's partial signal, (nf - 1) hop + 2048 samples
+// from sample t0 hop.  The final kernel adds, per output sample, the partials of the blocks
+// that cover it (block order), scales and divides by the window sum.
 struct IstftBlockArgs {
     const void* spec;   // [B, 1025, T] complex, f32 or bf16
     const float* w;
-    float* part;        // [B, nTB, span] block partials
+    float* part;        // [B, nTB, span] block partials, times 2048 / spectrum scale
     uint32_t T;
     FastDiv ntb;        // blocks per signal
     FastDiv hop;
     uint32_t span;      // (kTF - 1) hop + 2048: stride of a block's partial
     uint32_t blocks;    // B * nTB
-    int wvec;           // window is 8-byte aligned
-    float spec_scale;
 };
 
+// LDS slot of one frame, in floats: two runs of 513 bins (places up to 512 + 14), kHi apart, or
+// the frame's 2048 samples.
+constexpr int kHi = 528;
+constexpr int kSlotInv = 2 * (kHi + 528);
+static_assert(kSlotInv >= kN && kSlotInv >= kSlot, "a slot holds a frame and an exchange");
+
 template <int SDT>
-__device__ __forceinline__ float2 load_bin(const void* spec, int64_t i) {
-    if constexpr (SDT == F32) {
-        const f32x2 v = gld<MBRT_NT_STFT & 1>(static_cast<const f32x2*>(spec) + i);
-        return make_float2(v.x, v.y);
-    } else {
-        const uint32_t u = gld<MBRT_NT_STFT & 1>(static_cast<const uint32_t*>(spec) + i);
-        return make_float2(__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u));
-    }
+struct SpecElem {
+    typedef f32x2 T;
+};
+template <>
+struct SpecElem<BF16> {
+    typedef uint32_t T;
+};
+__device__ __forceinline__ float2 bin_f32(f32x2 v) { return make_float2(v.x, v.y); }
+__device__ __forceinline__ float2 bin_f32(uint32_t u) { return make_float2(bf16_lo(u), bf16_hi(u)); }
+
+// Inverse real split of bin k (with its mirror 1024 - k), times 2: Z[k] (MIRROR: Z[1024 - k])
+// from X[k], X[1024 - k] and W^-k = (c, s).
+template <bool MIRROR>
+__device__ __forceinline__ cf c2r_bin(float2 xk, float2 xg, float c, float s) {
+    const cf A{xk.x + xg.x, xk.y - xg.y}, Bv{xk.x - xg.x, xk.y + xg.y};
+    const cf Q = cmul(Bv, cf{c, s});
+    return MIRROR ? cf{A.x + Q.y, Q.x - A.y} : cf{A.x - Q.y, A.y + Q.x};
 }
 
-template <int TF, int SDT>
-__global__ __launch_bounds__(64 * TF) void istft_block_kernel(IstftBlockArgs a) {
-    constexpr int NT = 64 * TF;
-    __shared__ __attribute__((aligned(16))) float2 lds[TF * kSlot + kTwSlots];
-    float2* tw = lds + TF * kSlot;
+// Bound by its chain of phases: load, inverse split, FFT, window, overlap-add, with two
+// workgroups per CU by LDS.  Per frame 1,050 vector instructions (1,410 before) and 624 LDS cycles
+// (830 before), no bank conflicts.  Chunk [8, 1025, 801] f32: 29.6 -> 27.2 us; two signals of 620
+// frames, bf16, 156 workgroups: 12.4 -> 10.9.  Half slots as the STFT's, with the spectra and the
+// overlap-add in two rounds each (four workgroups per CU), ran 27.5 and 13.5.
+template <int SDT>
+__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(MBRT_ISTFT_WPE))) void istft_block_kernel(IstftBlockArgs a) {
+    typedef typename SpecElem<SDT>::T Elem;
+    __shared__ __attribute__((aligned(16))) float lds[kTF * kSlotInv + 2 * kTwSlots];
+    float2* tw = reinterpret_cast<float2*>(lds + kTF * kSlotInv);
     const uint32_t blk = xcd_runs<kXcdRunInv>(blockIdx.x, gridDim.x);
     uint32_t b, tb;
     fdivmod(blk, a.ntb, b, tb);
-    const uint32_t t0 = tb * TF;
-    const uint32_t nf = min((uint32_t)TF, a.T - t0);
-    // the twiddle loads go out with the spectrum's, one memory round trip for both
-    constexpr int kT = kTwHalf / NT;
-    float2 tv[kT];
-#pragma unroll
-    for (int k = 0; k < kT; ++k) tv[k] = reinterpret_cast<const float2*>(kTwiddles.v)[threadIdx.x + k * NT];
-    {
-        // transposed spectrum load: thread -> (frame tl, bins fr + 64 k, k = 0..15, and bin
-        // 1024 for fr = 0); all 16 (17) loads are in flight before the first LDS write
-        static_assert(NT / TF == 64, "64 bin rows per pass");
-        const int tl = threadIdx.x % TF, fr = threadIdx.x / TF;
-        if ((uint32_t)tl < nf) {
-            const int64_t idx = (int64_t)b * kBins * a.T + t0 + tl + (int64_t)fr * a.T;
-            const int64_t step = (int64_t)64 * a.T;
-            float2 X[17];
-#pragma unroll
-            for (int k = 0; k < 16; ++k) X[k] = load_bin<SDT>(a.spec, idx + k * step);
-            if (fr == 0) X[16] = load_bin<SDT>(a.spec, idx + 16 * step);
-            float2* slot = lds + tl * kSlot;
-#pragma unroll
-            for (int k = 0; k < 16; ++k)
-                slot[pad16(fr + 64 * k)] = make_float2(X[k].x * a.spec_scale, X[k].y * a.spec_scale);
-            if (fr == 0) slot[pad16(kN / 2)] = make_float2(X[16].x * a.spec_scale, X[16].y * a.spec_scale);
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < kT; ++k) tw[tw_pos(threadIdx.x + k * NT)] = tv[k];
-    __syncthreads();
+    const uint32_t t0 = tb * kTF;
+    const int nf = (int)min((uint32_t)kTF, a.T - t0);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if ((uint32_t)wave < nf) {
-        float2* slot = lds + wave * kSlot;
-        // inverse real split, in place: (X[k], X[1024 - k]) -> (Z[k], Z[1024 - k]) scaled by 2;
-        // Z[0] from the real parts of X[0] and X[1024] (their imaginary parts drop out).
-        cf x0{0.f, 0.f}, xn{0.f, 0.f};
-        if (lane == 0) {
-            x0 = lds_ld(slot, 0);
-            xn = lds_ld(slot, pad16(kN / 2));
-        }
+    const bool live = wave < nf;
+    // transposed spectrum load: thread -> (frame tl, bins fr + 64 j and their mirrors
+    // 1024 - fr - 64 j, j = 0..7, and bin 512 for fr = 0), all in flight before the first LDS
+    // write.  Frames past the block's last read that frame again.
+    const int tl = threadIdx.x % kTF, fr = threadIdx.x / kTF;
+    Elem lo[8], hi[8], mid;
+    {
+        const Elem* src = static_cast<const Elem*>(a.spec) + ((int64_t)b * kBins * a.T + t0 + min(tl, nf - 1));
+        const int64_t step = (int64_t)64 * a.T;
+        const Elem* pl = src + (int64_t)fr * a.T;
+        const Elem* ph = src + (int64_t)(kN / 2 - fr) * a.T;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int k = 1 + lane + 64 * q, gg = kN / 2 - k;
-            const cf xk = lds_ld(slot, pad16(k)), xg = lds_ld(slot, pad16(gg));
-            const cf A{xk.x + xg.x, xk.y - xg.y}, Bv{xk.x - xg.x, xk.y + xg.y};
-            const cf Q = cmul(Bv, twiddle<true>(tw, k));
-            lds_st(slot, pad16(k), cf{A.x - Q.y, A.y + Q.x});
-            lds_st(slot, pad16(gg), cf{A.x + Q.y, Q.x - A.y});
+        for (int j = 0; j < 8; ++j) {
+            lo[j] = gld<MBRT_NT_STFT & 1>(pl + j * step);
+            hi[j] = gld<MBRT_NT_STFT & 1>(ph - j * step);
         }
-        if (lane == 0) lds_st(slot, 0, cf{x0.x + xn.x, x0.x - xn.x});
-        wave_lds_sync();
+        mid = gld<MBRT_NT_STFT & 1>(src + (int64_t)512 * a.T);
+    }
+    const float2 t = reinterpret_cast<const float2*>(kFftTable.v)[min((int)threadIdx.x, kTwSlots - 1)];
+    // The spectra enter through LDS: X[k], k <= 512, at place k of the frame's slot and
+    // X[1024 - k] kHi further.  Places are rotated by the frame (p ^ 2 frame within 16), so that
+    // the 8 frames x 2 bins that 16 lanes write at a time fall on different banks.
+    float2* st = reinterpret_cast<float2*>(lds + tl * kSlotInv);
+    const int rt = tl << 1, fp = fr ^ rt;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        st[fp + 64 * j] = bin_f32(lo[j]);
+        st[kHi + fp + 64 * j] = bin_f32(hi[j]);
+    }
+    if (fr == 0) {
+        // the imaginary parts of bins 0 and 1024 drop out
+        st[rt].y = 0.0f;
+        st[kHi + rt].y = 0.0f;
+        st[512 + rt] = bin_f32(mid);
+        st[kHi + 512 + rt] = bin_f32(mid);
+    }
+    if (threadIdx.x < kTwSlots) tw[threadIdx.x] = t;
+    __syncthreads();
+    // Each lane forms the 16 bins of its first radix-16 pass, Z[l + 64 a]: for a < 8 from pair
+    // k = l + 64 a, for a = 15 - h as the mirror of pair k = m + 64 h, m = 64 - l.  Their twiddles
+    // W^-k have the angles a pi / 16 + th and (h + 1) pi / 16 - th, th that of S[l]; those
+    // past pi / 4 are swaps of the others.
+    float* slot = lds + wave * kSlotInv;
+    cf zA[4], zB[4], zC[4], zD[4];
+    if (live) {
+        const float2* xk = reinterpret_cast<const float2*>(slot);
+        constexpr float Kc[4] = {1.0f, 0.98078528040323044913f, 0.92387953251128675613f, 0.83146961230254523708f};
+        constexpr float Ks[4] = {0.0f, 0.19509032201612826785f, 0.38268343236508977173f, 0.55557023301960222474f};
+        constexpr float K4 = 0.70710678118654752440f;  // cos, sin of a pi / 16, a < 4, and pi / 4
+        const int rw = wave << 1, p = lane ^ rw, m = (64 - lane) ^ rw;
+        const cf w = lds_ld(tw, kTwS + lane);
+        const float c = w.x, n = -w.y;
         cf v[16];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) v[q] = lds_ld(slot, pad16(lane) + 68 * q);
-        fft1024<true>(v, slot, tw, lane);
-        // lane l holds 2048 * (x[2m], x[2m + 1]), m = l + 64a: the windowed frame goes back into
-        // the slot as 2048 consecutive floats
-        wave_lds_sync();
-        constexpr float kInvN = 1.0f / (float)kN;
+        for (int a = 0; a < 8; ++a) {
+            float cp, sp;  // a pi / 16 + th
+            if (a < 4) {
+                cp = a ? Kc[a] * c - Ks[a] * n : c;
+                sp = a ? Ks[a] * c + Kc[a] * n : n;
+            } else if (a == 4) {
+                cp = K4 * (c - n);
+                sp = K4 * (c + n);
+            } else {
+                cp = Ks[8 - a] * c - Kc[8 - a] * n;
+                sp = Kc[8 - a] * c + Ks[8 - a] * n;
+            }
+            v[a] = c2r_bin<false>(xk[p + 64 * a], xk[kHi + p + 64 * a], cp, sp);
+        }
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int m = lane + 64 * q;
-            float2 w;
-            if (a.wvec) w = reinterpret_cast<const float2*>(a.w)[m];
-            else w = make_float2(a.w[2 * m], a.w[2 * m + 1]);
-            slot[m] = make_float2(v[q].x * w.x * kInvN, v[q].y * w.y * kInvN);
+        for (int a = 1; a <= 8; ++a) {
+            float cm, sm;  // a pi / 16 - th
+            if (a < 4) {
+                cm = Kc[a] * c + Ks[a] * n;
+                sm = Ks[a] * c - Kc[a] * n;
+            } else if (a == 4) {
+                cm = K4 * (c + n);
+                sm = K4 * (c - n);
+            } else if (a < 8) {
+                cm = Ks[8 - a] * c + Kc[8 - a] * n;
+                sm = Kc[8 - a] * c - Ks[8 - a] * n;
+            } else {
+                cm = n;
+                sm = c;
+            }
+            v[16 - a] = c2r_bin<true>(xk[m + 64 * (a - 1)], xk[kHi + m + 64 * (a - 1)], cm, sm);
+        }
+        fft1024<true>(v, slot, tw, lane, zA, zB, zC, zD);
+    }
+    // zX[r] = 2048 (x[2i], x[2i + 1]), i = j + 256 r: the windowed frames go back to LDS, 2048 floats
+    // each, and the workgroup adds them, in frame order, to the block's partial (partial[u],
+    // u = s - t0 hop).
+    __syncthreads();  // the slots are no longer read
+    if (live) {
+        const int wm = lane ? lane : 64;
+        const int jb[4] = {lane, lane ? 256 - lane : 128, 128 + wm, 128 - wm};
+        float2* fs = reinterpret_cast<float2*>(lds + wave * kN);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const cf(&z)[4] = i == 0 ? zA : i == 1 ? zB : i == 2 ? zC : zD;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int k = jb[i] + 256 * r;
+                const float2 w = ld2_any(a.w + 2 * k);
+                fs[k] = make_float2(z[r].x * w.x, z[r].y * w.y);
+            }
         }
     }
     __syncthreads();
-    // overlap-add of the block's frames in frame order: partial[u], u = s - t0 hop
     const uint32_t hop = a.hop.d;
     const uint32_t span = (nf - 1) * hop + kN;
     float* part = a.part + (int64_t)blk * a.span;
-    for (uint32_t u = threadIdx.x; u < span; u += NT) {
-        const uint32_t jhi = min(nf - 1, fdiv(u, a.hop));
-        const uint32_t jlo = u >= (uint32_t)kN ? fdiv(u - kN, a.hop) + 1 : 0;
-        float acc = 0.0f;
-        for (uint32_t j = jlo; j <= jhi; ++j) acc += reinterpret_cast<const float*>(lds + j * kSlot)[u - j * hop];
-        gst<MBRT_NT_ISTFT & 2>(part + u, acc);
+    // chunks of 128 positions per wave and step, two per lane
+    for (uint32_t u0 = wave * 128; u0 < span; u0 += 128 * kTF) {
+        // frames that reach the chunk's first position, and its last
+        const uint32_t jlo = u0 >= (uint32_t)kN ? fdiv(u0 - kN, a.hop) + 1 : 0;
+        const uint32_t jhi = min((uint32_t)nf - 1, fdiv(u0 + 127, a.hop));
+        float acc0 = 0.0f, acc1 = 0.0f;
+        for (uint32_t j = jlo; j <= jhi; ++j) {
+            const float* f = lds + j * kN;
+            const uint32_t i0 = u0 - j * hop;  // wraps where the frame starts later
+            if (i0 <= (uint32_t)(kN - 128)) {  // the frame covers the whole chunk
+                acc0 += f[i0 + lane];
+                acc1 += f[i0 + lane + 64];
+            } else {
+                const uint32_t n0 = i0 + lane, n1 = n0 + 64;
+                const float x0 = f[min(n0, kN - 1u)], x1 = f[min(n1, kN - 1u)];
+                acc0 += n0 < (uint32_t)kN ? x0 : 0.0f;
+                acc1 += n1 < (uint32_t)kN ? x1 : 0.0f;
+            }
+        }
+        const uint32_t u = u0 + lane;
+        if (u < span) gst<MBRT_NT_ISTFT & 2>(part + u, acc0);
+        if (u + 64 < span) gst<MBRT_NT_ISTFT & 2>(part + u + 64, acc1);
     }
 }
 
@@ -684,6 +805,7 @@ struct IstftFinalArgs {
     uint32_t T;
     uint32_t valid;       // samples of the (trimmed) signal; out_len - valid zeros follow
     uint32_t offset;      // 1024 when centred
+    float scale;          // of the partials: spectrum scale / 2048
 };
 
 // One thread per output sample position, for every signal of the batch: the window sum
@@ -740,7 +862,7 @@ __global__ __launch_bounds__(256) void istft_final_kernel(IstftFinalArgs a) {
                     float acc = 0.0f;
                     if (v[0]) acc += p[k][0];
                     if (v[1]) acc += p[k][1];
-                    gst<(MBRT_NT_ISTFT & 4) ? 2 : 0>(a.out + (int64_t)(b0 + k) * a.out_len + so, ws > 1.0e-8f ? acc / ws : acc);
+                    gst<(MBRT_NT_ISTFT & 4) ? 2 : 0>(a.out + (int64_t)(b0 + k) * a.out_len + so, ws > 1.0e-8f ? acc * a.scale / ws : acc * a.scale);
                 }
             }
             continue;
@@ -754,7 +876,7 @@ __global__ __launch_bounds__(256) void istft_final_kernel(IstftFinalArgs a) {
                 const uint32_t nf = min((uint32_t)kTF, a.T - tb * kTF);
                 if (u < (nf - 1) * hop + kN) acc += gld<MBRT_NT_ISTFT & 1>(pb + (int64_t)tb * a.span + u);
             }
-            gst<(MBRT_NT_ISTFT & 4) ? 2 : 0>(a.out + (int64_t)b * a.out_len + so, ws > 1.0e-8f ? acc / ws : acc);
+            gst<(MBRT_NT_ISTFT & 4) ? 2 : 0>(a.out + (int64_t)b * a.out_len + so, ws > 1.0e-8f ? acc * a.scale / ws : acc * a.scale);
         }
     }
 }
@@ -831,14 +953,24 @@ int mbrt_stft(const float* signal, const float* window, float* out, int64_t batc
     a.ntb = make_fastdiv((uint32_t)ntb);
     a.hop = (int)hop;
     a.offset = center ? kN / 2 : 0;
-    a.norm = normalized ? 1.0f / std::sqrt((float)kN) : 1.0f;
-    a.wvec = aligned(window, 8) ? 1 : 0;
-    a.xvec = aligned(signal, 16) ? 1 : 0;
-    // window + span (+ up to 6 floats of float4 alignment) within the kTF frame slots
-    a.staged = kN + (kTF - 1) * hop + kN + 6 <= 2 * kTF * kSlot ? 1 : 0;
-    const int64_t blocks = batch * ntb;
-    MBRT_REQUIRE(blocks < kMaxGridX, MBRT_E_SHAPE, "%s: too many frames", op);
-    hipLaunchKernelGGL((stft_kernel<kTF>), dim3((unsigned)blocks), dim3(64 * kTF), 0, as_stream(stream), a);
+    a.scale = normalized ? 0.5f / std::sqrt((float)kN) : 0.5f;
+    // what the kTF frame slots hold: the window and the span (hops up to 658), the span alone (up to
+    // 950), or neither: each wave then reads its frame from memory
+    const int64_t span = (kTF - 1) * hop + kN;
+    a.staged = kN + span <= kTF * kSlot ? 2 : span <= kTF * kSlot ? 1 : 0;
+    const int64_t groups = batch * ntb;
+    MBRT_REQUIRE(groups < kMaxGridX, MBRT_E_SHAPE, "%s: too many frames", op);
+    // A CU that gets one group more than the others sets the time, so the groups left over after
+    // every CU has the same number are taken by two workgroups each, four frames apiece, when
+    // they would fill at most half of the CUs (beyond that the halves cost more than the even
+    // spread gives: each stages 3/4 of the whole group's samples).  Chunk of 808 groups, 40 left over:
+    // 22.1 -> 20.8 us; 7 groups (0.5 s of mono) 7.4 -> 6.5; 632 groups, hop 1000: 13.5 -> 13.0.
+    // Parts of 2 and 1 frames: 21.0 and 23.2 on the chunk.
+    const int64_t cus = cu_count(), rem = groups % cus;
+    const int64_t parts = 2 * rem <= cus ? rem : 0;
+    a.whole = (uint32_t)(groups - parts);
+    const int64_t blocks = a.whole + parts * (kTF / kSub);
+    hipLaunchKernelGGL(stft_kernel, dim3((unsigned)blocks), dim3(kNT), 0, as_stream(stream), a);
     return check_launch(op);
 }
 
@@ -934,12 +1066,8 @@ int istft_impl(const char* op, const void* spec, int spec_dtype, const float* wi
     ba.hop = make_fastdiv((uint32_t)hop);
     ba.span = (uint32_t)((kTF - 1) * hop + kN);
     ba.blocks = (uint32_t)(batch * ntb);
-    ba.wvec = aligned(window, 8) ? 1 : 0;
-    ba.spec_scale = normalized ? std::sqrt((float)kN) : 1.0f;
-    if (spec_dtype == F32)
-        hipLaunchKernelGGL((istft_block_kernel<kTF, F32>), dim3(ba.blocks), dim3(64 * kTF), 0, st, ba);
-    else
-        hipLaunchKernelGGL((istft_block_kernel<kTF, BF16>), dim3(ba.blocks), dim3(64 * kTF), 0, st, ba);
+    if (spec_dtype == F32) hipLaunchKernelGGL(istft_block_kernel<F32>, dim3(ba.blocks), dim3(kNT), 0, st, ba);
+    else hipLaunchKernelGGL(istft_block_kernel<BF16>, dim3(ba.blocks), dim3(kNT), 0, st, ba);
     s = check_launch(op);
     if (s != MBRT_OK) return s;
     IstftFinalArgs fa{};
@@ -955,6 +1083,7 @@ int istft_impl(const char* op, const void* spec, int spec_dtype, const float* wi
     fa.T = (uint32_t)frames;
     fa.valid = (uint32_t)std::min<int64_t>(out_len, center ? full - kN : full);
     fa.offset = center ? kN / 2 : 0;
+    fa.scale = (normalized ? std::sqrt((float)kN) : 1.0f) / (float)kN;
     hipLaunchKernelGGL(istft_final_kernel, dim3((unsigned)grid_for(out_len, 256)), dim3(256), 0, st, fa);
     return check_launch(op);
 }

@@ -57,6 +57,43 @@ def test_stft_shapes(orc, dev, B, L, hop, center, normalized, win):
     print("stft errors", assert_close(to_host(out, F32), ref, F32, "stft", den=den))
 
 
+# the STFT's staging forms at their limits (window and span, span alone, frame by frame), odd hops
+# and rows, frame counts that leave a group's parts empty or ragged, groups all in parts (at most
+# half as many as CUs) and all whole (1037 frames: 130 groups)
+@pytest.mark.parametrize("B,frames,hop,normalized", [
+    (1, 17, 657, False), (1, 21, 658, True), (2, 13, 659, False), (1, 9, 949, False), (1, 12, 950, True),
+    (1, 11, 951, False), (3, 5, 441, True), (2, 4, 333, False), (1, 1, 441, False), (1, 1037, 101, False),
+    (1, 1025, 2, False)])
+def test_stft_staging_and_parts(orc, dev, B, frames, hop, normalized):
+    say(f"stft B={B} frames={frames} hop={hop} normalized={normalized}")
+    L = (frames - 1) * hop + 1 if frames > 1 else 300
+    x = orc.randn((B, L), seed=0x4D425200BA, stream=frames)
+    w = _window(orc, "rand")
+    out = mbrt.stft(to_dev(x, F32), to_dev(w, F32), hop, True, normalized)
+    torch.cuda.synchronize()
+    assert out.shape[2] == (L // hop + 1)
+    assert_close(to_host(out, F32), orc.stft(x, w, hop, True, normalized), F32, "stft",
+                 den=orc.stft_den(x, w, hop, True, normalized))
+
+
+# the overlap-add's chunks of 128 positions: hops at their edges, hops with gaps between frames,
+# one frame, a last block of one and of seven frames; non-zero imaginary parts at bins 0 and 1024
+@pytest.mark.parametrize("dt", [F32, BF16])
+@pytest.mark.parametrize("B,T,hop,center,normalized", [
+    (1, 1, 441, False, False), (2, 9, 127, False, True), (1, 15, 128, True, False), (1, 8, 129, False, False),
+    (1, 10, 1, False, False), (2, 7, 1921, False, True), (1, 9, 2048, False, False), (1, 12, 2100, False, False),
+    (1, 17, 441, True, True)])
+def test_istft_overlap_add_edges(orc, dev, B, T, hop, center, normalized, dt):
+    say(f"istft B={B} T={T} hop={hop} center={center} normalized={normalized} dt={dt}")
+    s = orc.randn((B, 1025, T, 2), seed=0x4D425200BB, stream=T)
+    s = s if dt == F32 else orc.from_f32(s, dt)
+    w = _window(orc, "rand")
+    y = mbrt.istft(to_dev(s, dt), to_dev(w, F32), hop, center, normalized)
+    torch.cuda.synchronize()
+    assert_close(to_host(y, F32), orc.istft(s, dt, w, hop, center, normalized, -1), F32, "istft",
+                 den=orc.istft_den(s, dt, w, hop, center, normalized, -1))
+
+
 @pytest.mark.parametrize("shift", [1, 2, 3])
 def test_stft_unaligned_buffers(orc, dev, shift):
     """Signal and window that start off a 16-byte (window: 8-byte) boundary."""
