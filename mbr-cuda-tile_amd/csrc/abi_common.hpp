@@ -37,6 +37,9 @@ int check_launch(const char* op);
 // Compute units of the current device (queried once per device), for persistent grids.
 int cu_count();
 
+// Whether a kernel reads `bytes` of streaming input non-temporally where its policy says so.
+inline int cold_input(int64_t bytes, int64_t limit = MBRT_HOT_BYTES) { return bytes > limit ? 1 : 0; }
+
 // Largest grid.x we launch (2^31 - 1 allowed on AMD, but keep index math in 32 bits
 // where kernels assume it).
 constexpr int64_t kMaxGridX = 0x7fffffffLL;

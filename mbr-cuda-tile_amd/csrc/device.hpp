@@ -354,6 +354,22 @@ __device__ __forceinline__ void gst(T* p, T v) {
 
 // 16 bytes at an address aligned to A bytes only (A = 4 or 2): one dwordx4 access, which
 // global memory takes at any alignment (unaligned access mode, the default of HSA code).
+// Issues a kernel's streaming loads, f(std::integral_constant<int, policy>), by policy NT when
+// `cold` (uniform), else with ordinary loads.  The empty asm statements keep the compiler from
+// merging the two branches' loads into one set, which drops the non-temporal bit.
+template <int NT, class F>
+__device__ __forceinline__ void load_by(int cold, F f) {
+    if constexpr ((NT & 1) == 0) {
+        f(std::integral_constant<int, NT>());
+    } else if (cold) {
+        asm volatile("" ::: "memory");
+        f(std::integral_constant<int, NT>());
+        asm volatile("" ::: "memory");
+    } else {
+        f(std::integral_constant<int, (NT & 2)>());
+    }
+}
+
 template <int A>
 struct AnyVec;
 template <> struct AnyVec<4> { typedef uint32_t T __attribute__((ext_vector_type(4), aligned(4))); };

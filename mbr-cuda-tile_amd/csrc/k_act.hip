@@ -123,6 +123,7 @@ struct GluArgs {
     int64_t rows, half;
     int64_t groups;   // rows * half / VE
     FastDiv gpr;      // groups per row = half / VE
+    int cold;         // the input is too large to be cached
     int fb;           // bf16 intermediates (element kernel; the vector kernel takes FB)
 };
 
@@ -131,14 +132,17 @@ __global__ __launch_bounds__(kThreads) void glu_vec_kernel(GluArgs a) {
     constexpr int VE = (XDT == F32 || ODT == F32) ? 4 : 8;
     const int64_t base = (int64_t)blockIdx.x * (kThreads * kUGlu) + threadIdx.x;
     Vec<XDT, VE> xv[kUGlu], gv[kUGlu];
+    load_by<MBRT_NT_GLU>(a.cold, [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
 #pragma unroll
-    for (int u = 0; u < kUGlu; ++u) {
-        uint32_t row, c;
-        fdivmod((uint32_t)clamp_group(base + u * kThreads, a.groups), a.gpr, row, c);
-        const int64_t in0 = (int64_t)row * (2 * a.half) + (int64_t)c * VE;
-        xv[u].template load<MBRT_NT_GLU>(a.x, in0);
-        gv[u].template load<MBRT_NT_GLU>(a.x, in0 + a.half);
-    }
+        for (int u = 0; u < kUGlu; ++u) {
+            uint32_t row, c;
+            fdivmod((uint32_t)clamp_group(base + u * kThreads, a.groups), a.gpr, row, c);
+            const int64_t in0 = (int64_t)row * (2 * a.half) + (int64_t)c * VE;
+            xv[u].template load<NT>(a.x, in0);
+            gv[u].template load<NT>(a.x, in0 + a.half);
+        }
+    });
 #pragma unroll
     for (int u = 0; u < kUGlu; ++u) {
         const int64_t g = base + u * kThreads;
@@ -182,6 +186,7 @@ struct GateArgs {
     FastDiv n_div;     // N
     FastDiv sb_div;    // MBRT_GATE_TPW * groups per token
     int tpw_ok;        // B * N is a multiple of MBRT_GATE_TPW
+    int cold;          // the attention values are too large to be cached
     int fb;            // bf16 intermediates (element kernel; the vector kernel takes FB)
 };
 
@@ -194,7 +199,7 @@ __global__ __launch_bounds__(kThreads) void gate_merge_vec_kernel(GateArgs a) {
     const int64_t base = chunk * (kThreads * kUGate) + threadIdx.x;
     Vec<ADT, VE> av[kUGate];
     float gl[kUGate];
-    int64_t dst[kUGate];
+    int64_t dst[kUGate], srcs[kUGate];
 #pragma unroll
     for (int u = 0; u < kUGate; ++u) {
         const uint32_t g = (uint32_t)clamp_group(base + u * kThreads, a.groups);
@@ -225,9 +230,13 @@ __global__ __launch_bounds__(kThreads) void gate_merge_vec_kernel(GateArgs a) {
             }
             dst[u] = (int64_t)g * VE;
         }
-        av[u].template load<MBRT_NT_GATE>(a.attn, src);
+        srcs[u] = src;
         gl[u] = ld1<GDT>(a.gate, (int64_t)token * a.H + h);
     }
+    load_by<MBRT_NT_GATE>(a.cold, [&](auto nt) {
+#pragma unroll
+        for (int u = 0; u < kUGate; ++u) av[u].template load<decltype(nt)::value>(a.attn, srcs[u]);
+    });
 #pragma unroll
     for (int u = 0; u < kUGate; ++u) {
         const int64_t g = base + u * kThreads;
@@ -360,6 +369,7 @@ int mbrt_glu_last_dim(const void* x, int x_dtype, void* out, int out_dtype, int6
     if (vec) {
         a.groups = rows * half_dim / ve;
         a.gpr = make_fastdiv((uint32_t)(half_dim / ve));
+        a.cold = cold_input(2 * rows * half_dim * dt_size(x_dtype), MBRT_HOT_BYTES_ACT);
         with_dt(x_dtype, [&](auto xt) {
             with_dt(out_dtype, [&](auto ot) {
                 constexpr int X = decltype(xt)::value, O = decltype(ot)::value;
@@ -416,6 +426,7 @@ int mbrt_sigmoid_gate_merge(const void* attn, int attn_dtype, const void* gate, 
         a.n_div = make_fastdiv((uint32_t)N);
         a.sb_div = make_fastdiv((uint32_t)(MBRT_GATE_TPW * H * D / ve));
         a.tpw_ok = (B * N) % MBRT_GATE_TPW == 0 ? 1 : 0;
+        a.cold = cold_input(total * dt_size(attn_dtype));
         with_dt(attn_dtype, [&](auto at) {
             with_dt(gate_dtype, [&](auto gt) {
                 with_dt(out_dtype, [&](auto ot) {

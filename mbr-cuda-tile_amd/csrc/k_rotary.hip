@@ -116,6 +116,7 @@ struct SplitArgs {
     const void* sinp;
     int64_t B, N, H, D, outN;
     int fb;  // bf16 intermediates (scalar kernel; the vector kernel takes FB)
+    int cold;  // qkv is too large to be cached
 };
 
 // One thread per VE-element group of the [B, H, outN, D] outputs (q, k and v together);
@@ -137,9 +138,12 @@ __global__ __launch_bounds__(kThreads) void split_qkv_vec_kernel(SplitArgs a, ui
     const int64_t t = nn * (a.D / 2) + (int64_t)c * (VE / 2);
     Vec<IDT, VE> vq, vk, vv;
     Vec<TDT, VE / 2> cv, sv;
-    vq.template load<MBRT_NT_ROT>(a.qkv, src);
-    vk.template load<MBRT_NT_ROT>(a.qkv, src + a.H * a.D);
-    vv.template load<MBRT_NT_ROT>(a.qkv, src + 2 * a.H * a.D);
+    load_by<MBRT_NT_ROT>(a.cold, [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
+        vq.template load<NT>(a.qkv, src);
+        vk.template load<NT>(a.qkv, src + a.H * a.D);
+        vv.template load<NT>(a.qkv, src + 2 * a.H * a.D);
+    });
     cv.load(a.cosp, t);
     sv.load(a.sinp, t);
     float xq[VE], xk[VE], xv[VE], cs[VE / 2], sn[VE / 2];
@@ -322,6 +326,7 @@ int mbrt_split_qkv_heads_rotary(const void* qkv, int qkv_dtype, const void* cos_
                      tab_al && groups < (1ll << 31);
     if (vec) {
         const dim3 grid((unsigned)ceil_div(groups, kThreads));
+        a.cold = cold_input(3 * B * N * H * D * dt_size(qkv_dtype));
         const FastDiv gpr = make_fastdiv((uint32_t)(D / ve)), od = make_fastdiv((uint32_t)out_N),
                       hd = make_fastdiv((uint32_t)H);
         with_dt(qkv_dtype, [&](auto it) {

@@ -35,6 +35,7 @@ struct SmArgs {
     int cols;
     float scale_log2e;
     float scale;  // bf16-intermediates mode: the scale is applied (and rounded) on its own
+    int cold;     // the input is too large to be cached: its loads go by the kernels' policy
 };
 
 // Bf16-intermediates mode (scale_softmax_bf16_to_bf16_kernel in full-bf16 mode,
@@ -95,11 +96,13 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_kernel(SmArgs a) {
 // as above but fed from LDS, writing the probabilities back over their inputs, phase 3
 // stores the span.  In-place calls are safe: the whole span is in LDS before its first
 // store.
-template <int IDT, int ODT, int G, int NM, int RPG, bool FB>
+// HOT: the input is small enough to be cached (see MBRT_HOT_BYTES) and loaded by ordinary
+// loads.  (An instance of its own: the choice at run time cost the time softmax 0.2 %.)
+template <int IDT, int ODT, int G, int NM, int RPG, bool FB, bool HOT = false>
 __global__ __launch_bounds__(kThreads) void softmax_staged_kernel(SmArgs a) {
     constexpr int RB = RPG * kThreads / G;
     // rows of more than 128 elements (groups of 32 or 64 lanes) have their own cache policy
-    constexpr int NT = G >= 32 ? MBRT_NT_SML : MBRT_NT_SMS;
+    constexpr int NT = (G >= 32 ? MBRT_NT_SML : MBRT_NT_SMS) & (HOT ? 2 : 3);
     constexpr int VI = 16 / DtSize<IDT>::value, VO = 16 / DtSize<ODT>::value;
     constexpr int CAP = RB * G * NM;  // elements of LDS (RB rows of at most G*NM elements)
     constexpr int KI = (CAP / VI + kThreads - 1) / kThreads, KO = (CAP / VO + kThreads - 1) / kThreads;
@@ -261,11 +264,13 @@ __global__ __launch_bounds__(kThreads) void softmax_pair_kernel(SmArgs a) {
     for (int64_t chunk = blockIdx.x; chunk < chunks; chunk += gridDim.x) {
     const int64_t p0 = chunk * (kGroups * U) + (threadIdx.x >> 4);
     Vec<DT, 8> x[U];
+    load_by<MBRT_NT_SMP>(a.cold, [&](auto nt) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int64_t p = min(p0 + u * kGroups, pairs - 1);
-        x[u].template load<MBRT_NT_SMP>(a.in, (p * nv + vi) * 8);
-    }
+        for (int u = 0; u < U; ++u) {
+            const int64_t p = min(p0 + u * kGroups, pairs - 1);
+            x[u].template load<decltype(nt)::value>(a.in, (p * nv + vi) * 8);
+        }
+    });
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         float z[8];
@@ -348,8 +353,15 @@ void launch_staged(const SmArgs& a, bool fb, hipStream_t st) {
         }
     }
     with_dt(a.odt, [&](auto ot) {
-        hipLaunchKernelGGL((softmax_staged_kernel<IDT, decltype(ot)::value, G, NM, RPG, false>), grid, dim3(kThreads),
-                           0, st, a);
+        constexpr int O = decltype(ot)::value;
+        if constexpr (IDT == O) {
+            if (!a.cold) {
+                hipLaunchKernelGGL((softmax_staged_kernel<IDT, O, G, NM, RPG, false, true>), grid, dim3(kThreads), 0, st,
+                                   a);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((softmax_staged_kernel<IDT, O, G, NM, RPG, false>), grid, dim3(kThreads), 0, st, a);
     });
 }
 
@@ -459,6 +471,7 @@ int mbrt_softmax_rows(const void* in, int in_dtype, void* out, int out_dtype, in
     a.cols = (int)cols;
     a.scale_log2e = scale * kLog2e;
     a.scale = scale;
+    a.cold = cold_input(rows * cols * dt_size(in_dtype));
     // bf16 intermediates: bf16 -> bf16 rows, as in the reference
     const bool fb = bf16_intermediates() && in_dtype == BF16 && out_dtype == BF16;
     hipStream_t st = as_stream(stream);

@@ -9,6 +9,21 @@
 //             policies 0..3 per kernel, the best kept; differences under ~3 % are noise.
 #pragma once
 
+// Inputs of up to MBRT_HOT_BYTES bytes are read with ordinary loads whatever the policy says:
+// an input that small has usually just been written and still sits in the 256 MB MALL (or an
+// L2), which non-temporal loads make no use of.  Each kernel over two cycled buffer sets: split +
+// rotary of 18.6 MB 8.35 -> 6.21 us, gate merge of 12.3 MB 6.19 -> 4.28, permute of 18.5 MB
+// 8.24 -> 7.04, f32 softmax [4000, 801] 5.11 -> 4.58, bf16 rows of 60 columns 2.87 -> 2.64.  Larger
+// inputs gain as much while they are warm (split of 37 MB 14.5 -> 12.1), but in a chain of calls they
+// are cold by then and lose: the token step of 401 frames 61.6 -> 62.9 us with 40 MB as the limit.
+// RMSNorm and GLU, whose second operands come from further back, take MBRT_HOT_BYTES_ACT:
+// with 20 MB the token step of 201 frames ran 33.9 -> 34.9 us over three buffer sets.
+#ifndef MBRT_HOT_BYTES
+#define MBRT_HOT_BYTES (20ll << 20)
+#endif
+#ifndef MBRT_HOT_BYTES_ACT
+#define MBRT_HOT_BYTES_ACT (12ll << 20)
+#endif
 #ifndef MBRT_NT_RMS
 #define MBRT_NT_RMS 3    // residual add + RMSNorm: x, residual, sum, normed
 #endif

@@ -338,6 +338,56 @@ def test_reductions(orc, dev):
         assert_bitexact(to_host(out, F32), orc.reduce_general(x, 1, op), f"general reduce {op}")
 
 
+# ---- cache policy by input size ------------------------------------------------------------
+
+# Inputs just below and above the sizes where the streaming kernels change their load policy
+# (12 MB for RMSNorm and GLU, 20 MB for the others) give the same results: each call over the
+# large input against calls over its two halves
+def test_load_policy_changes_no_result(dev):
+    say("load policy: whole inputs of 12..24 MB against their halves")
+    g = torch.Generator(device="cuda").manual_seed(11)
+    rnd = lambda *s, dt=torch.bfloat16: torch.randn(s, generator=g, device="cuda").to(dt)  # noqa: E731
+    gamma = torch.ones(384, device="cuda")
+
+    def halves(fn, n, *xs):  # fn(*inputs) -> output, rows first
+        whole = fn(*xs)
+        parts = torch.cat([fn(*(x[:n].contiguous() for x in xs)), fn(*(x[n:].contiguous() for x in xs))])
+        torch.cuda.synchronize()
+        assert torch.equal(whole, parts), fn.__name__
+
+    def rms(x, r):
+        return mbrt.residual_add_rms_norm(x, r, gamma, torch.empty_like(x), torch.empty_like(x), 19.6)
+
+    def glu(x):
+        return mbrt.glu(x, torch.empty((x.shape[0], x.shape[1] // 2), dtype=x.dtype, device="cuda"))
+
+    def gate(x, l):
+        return mbrt.gate_merge(x, l, torch.empty((x.shape[0], x.shape[2], 512), dtype=x.dtype, device="cuda"))
+
+    def softmax(x):
+        return mbrt.softmax(x, torch.empty_like(x))
+
+    def permute(x):
+        return mbrt.strided_copy(x.permute(0, 2, 1, 3), torch.empty((x.shape[0], x.shape[2], x.shape[1], x.shape[3]),
+                                                                    dtype=x.dtype, device="cuda"))
+
+    cos, sin = (torch.from_numpy(t).to("cuda") for t in mbrt.rotary_tables(131, 64))
+
+    def split(x):
+        q, k, v = (torch.empty((x.shape[0], 8, 131, 64), dtype=x.dtype, device="cuda") for _ in range(3))
+        mbrt.split_qkv_rotary(x, cos, sin, q, k, v, 8)
+        return torch.stack((q, k, v), 1)
+
+    halves(rms, 4100, rnd(8300, 384), rnd(8300, 384))
+    halves(glu, 1024, rnd(2052, 3072))
+    halves(gate, 12, rnd(26, 8, 801, 64), rnd(26, 801, 8))
+    halves(softmax, 6552, rnd(13128, 801))
+    halves(softmax, 3276, rnd(6564, 801, dt=torch.float32))
+    halves(softmax, 90000, rnd(180000, 60))
+    halves(permute, 2, rnd(4, 120, 60, 384))
+    halves(split, 26, rnd(53, 131, 1536))
+
+
 # ---- normalisation ------------------------------------------------------------------------
 
 def test_residual_rmsnorm_bl1_full(orc, dev):
