@@ -50,10 +50,6 @@ constexpr int kBufferDword3 = 0x00020000;
 #ifndef MBRT_ATTN_PRIO_PAIR
 #define MBRT_ATTN_PRIO_PAIR 1  // the bf16-pair mode raises wave priority around its MFMA blocks
 #endif
-#ifndef MBRT_ATTN_QS2_MIN
-#define MBRT_ATTN_QS2_MIN 1  // 32 queries per wave when n_q exceeds this many 64-query blocks
-#endif
-
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -679,6 +675,29 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(HEA
     }
 }
 
+// Whether 16 queries per wave (64 per workgroup) beat 32 (128), for n_q > 64.  32 use each K and V
+// fragment read from LDS twice and do the same work in fewer instructions, so they win once
+// every CU has many workgroups.  Below that a call takes as long as the CU with the most of
+// them, c2 workgroups of 128 queries or c1 of 64 (about half as long each), and 64-query
+// ones also pad less.  Measured (us, 32 -> 16 queries per wave, P pair):
+//   c2 = 1                [8, 801] 18.7 -> 12.8, [60, 401] 12.6 -> 10.8, [120, 200] 9.0 -> 8.0
+//   c1 <= 2 c2 - c2 / 4   [48, 801] (2, 3) 27.9 -> 23.0, [480, 150] (4, 6) 17.1 -> 14.8,
+//                         [480, 300] (6, 10) 32.1 -> 29.8, [480, 401] (8, 14) 51.9 -> 48.8
+//   above                 [60, 801] (2, 4) 25.9 -> 27.1, [120, 1601] (7, 13) 140 -> 149
+// The single-P modes, with less arithmetic per fragment, need half the margin more: [240, 401]
+// (4, 7) 31.0 -> 29.3 as a pair but 22.1 -> 23.1 fast; [48, 801] 21.2 -> 17.8 fast.  A tie (c1 =
+// 2 c2 <= 4) goes to 16 where there are few key tiles and the 64-query workgroups are mostly
+// full: [480, 101] fast 8.4 -> 7.9, [480, 128] 9.4 -> 8.5, but [480, 70] pair 7.7 -> 8.1.
+bool narrow_queries(int64_t BH, int64_t n_q, int64_t n_k, bool pair) {
+    const int64_t cus = cu_count();
+    const int64_t t1 = ceil_div(n_q, kQBlock), t2 = ceil_div(n_q, 2 * kQBlock);
+    const int64_t c1 = ceil_div(BH * t1, cus), c2 = ceil_div(BH * t2, cus);
+    if (c2 == 1) return true;
+    if (c2 > 8) return false;
+    if (c1 + ceil_div(c2, pair ? 4 : 2) <= 2 * c2) return true;
+    return c2 == 2 && n_k <= 4 * kKeys && 4 * n_q >= 3 * kQBlock * t1;
+}
+
 }  // namespace
 }  // namespace mbrt
 
@@ -751,8 +770,7 @@ int mbrt_attention_ex(const void* q, const void* k, const void* v, int dtype, in
     a.gate = gate;
     a.gdt = gate_dtype;
     a.glogit = gate_is_logit ? 1 : 0;
-    // two query sub-blocks per wave once a (b, h) has more than one workgroup of queries
-    const int qs = n_q > kQBlock * MBRT_ATTN_QS2_MIN ? 2 : 1;
+    const int qs = n_q <= kQBlock || narrow_queries(BH, n_q, n_k, p_precision == MBRT_ATTN_P_PAIR) ? 1 : 2;
     a.qtiles = (uint32_t)ceil_div(n_q, (int64_t)kQBlock * qs);
     MBRT_REQUIRE(BH * a.qtiles < (int64_t(1) << 31), MBRT_E_SHAPE, "%s: too many tiles", op);
     a.nbh = (uint32_t)BH;

@@ -1056,6 +1056,44 @@ def test_attention_short_heads_persistent(orc, dev, BH, nq, nk, pm, odt):
                       flips=4)
 
 
+# 32 queries per wave (many heads) against 16 (few), which the shapes above are checked with: the
+# same results bit for bit, for query counts around the edges of both workgroups and key counts
+# around the tiles'; n_q != n_k; every precision; plain and from the fused projection
+@pytest.mark.parametrize("pm", [mbrt.ATTN_P_PAIR, mbrt.ATTN_P_BF16, mbrt.ATTN_P_BF16_FAST])
+@pytest.mark.parametrize("nq,nk", [(65, 65), (128, 64), (129, 130), (97, 200), (193, 63), (256, 1)])
+def test_attention_wide_and_narrow_workgroups(dev, nq, nk, pm):
+    BH = 2304
+    say(f"attention wide/narrow BH={BH} nq={nq} nk={nk} P mode {pm}")
+    g = torch.Generator(device="cuda").manual_seed(nq * 300 + nk)
+    q, k, v = (torch.randn((BH, n, 64), generator=g, device="cuda").to(torch.bfloat16) * s
+               for n, s in ((nq, 2.0), (nk, 1.0), (nk, 1.0)))
+    out = torch.empty((BH, nq, 64), device="cuda")
+    mbrt.attention(q, k, v, out, p_precision=pm)
+    few = torch.empty((24, nq, 64), device="cuda")
+    for b in (0, 1140, BH - 24):
+        mbrt.attention(q[b:b + 24], k[b:b + 24], v[b:b + 24], few, p_precision=pm)
+        torch.cuda.synchronize()
+        assert torch.equal(out[b:b + 24], few), f"heads {b}.."
+
+
+def test_attention_bnhd_wide_and_narrow_workgroups(dev):
+    say("attention_bnhd wide/narrow [288, 133] x 8 heads, rotary and gate")
+    B, N, H = 288, 133, 8
+    g = torch.Generator(device="cuda").manual_seed(5)
+    qkv = torch.randn((B, N, 3, H, 64), generator=g, device="cuda").to(torch.bfloat16)
+    gate = torch.randn((B, N, H), generator=g, device="cuda").to(torch.bfloat16)
+    cos, sin = (torch.from_numpy(t).to("cuda") for t in mbrt.rotary_tables(N, 64))
+
+    def run(b0, b1):
+        x = qkv[b0:b1]
+        return mbrt.attention_bnhd(x[:, :, 0], x[:, :, 1], x[:, :, 2], cos=cos, sin=sin, gate=gate[b0:b1].contiguous())
+
+    whole = run(0, B)
+    torch.cuda.synchronize()
+    for b in (0, 150, B - 3):
+        assert torch.equal(whole[b:b + 3], run(b, b + 3)), f"batch {b}.."
+
+
 def test_attention_p_bf16_fast_known_answer(orc, dev):
     """v = 1: the output and the row sum add the same rounded P in the same order, so every
     output is 1 up to the final division (one f32 rounding)."""
