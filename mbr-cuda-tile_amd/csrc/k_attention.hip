@@ -197,7 +197,7 @@ __device__ __forceinline__ float xor_sum(float x) {
 }
 
 // QS = 16-query sub-blocks per wave (1 or 2): every K and V^T fragment read from LDS
-// feeds QS MFMAs, so longer sequences use QS = 2 (128 queries per workgroup).
+// feeds QS MFMAs, so QS = 2 (128 queries per workgroup) is the wider form (narrow_queries).
 // PM = precision of P in the second product: MBRT_ATTN_P_PAIR (P as a bf16 hi + lo pair,
 // f32 accuracy, lazy max), MBRT_ATTN_P_BF16 (the reference's arithmetic,
 // src/mbr_time_attention_cutile.cu:160-180: the running max moves every 64-key tile, P is
