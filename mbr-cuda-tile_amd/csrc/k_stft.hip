@@ -123,9 +123,16 @@ constexpr TwiddleTable make_twiddles() {
 //   V  W256^(q n),  q = 1..3, n = k + 16 r < 64   pass 2, between its two radix-4 steps
 //   U  W64^(q k),   q = 1..3, k < 16              pass 2, on its inputs
 //   P  W1024^(q l), q = 1..3, l <= 64             pass 3 (further ones by reflection)
-//   S  W2048^l,     l <= 64                       real split (further ones by rotation)
-constexpr int kTwV = 0, kTwU = kTwV + 3 * 64, kTwP = kTwU + 3 * 16, kTwS = kTwP + 3 * 65, kTwSlots = kTwS + 65;
-static_assert(kTwSlots <= kNT, "one twiddle per thread");
+//   S  W2048^l,     l <= 64, inverse l <= 256     real split (further ones by rotation, in the
+//                                                 inverse by swaps)
+// Error of the result (relative, rms, against 64 bits; twelve inputs, hops 256 to 1000), beside
+// 1.30e-7 and 1.38e-7 (STFT, iSTFT) of the form that formed pass 2's twiddles from products:
+// 1.28e-7 and 1.36e-7.  The inverse with S rotated too: 1.40e-7 at 32.3 us a call on the chunk
+// instead of 32.5, which is why it reads all of S.  With P up to l = 192 as well, and all of S,
+// the STFT has 1.26e-7 but takes 19.1 us instead of 18.3.
+constexpr int kTwV = 0, kTwU = kTwV + 3 * 64, kTwP = kTwU + 3 * 16, kTwS = kTwP + 3 * 65;
+constexpr int kTwFwd = kTwS + 65, kTwSlots = kTwS + 257;  // slots of the STFT, and of the iSTFT
+static_assert(kTwFwd <= kNT && kTwSlots > kNT && kTwSlots <= 2 * kNT, "one twiddle per thread, and two");
 
 struct FftTable {
     float v[2 * kTwSlots];
@@ -142,7 +149,7 @@ constexpr FftTable make_fft_table() {
         for (int k = 0; k < 16; ++k) put(kTwU + (q - 1) * 16 + k, 32 * q * k);
         for (int l = 0; l <= 64; ++l) put(kTwP + (q - 1) * 65 + l, 2 * q * l);
     }
-    for (int l = 0; l <= 64; ++l) put(kTwS + l, l);
+    for (int l = 0; l <= 256; ++l) put(kTwS + l, l);
     return t;
 }
 
@@ -405,7 +412,7 @@ template <int KS, int KH, bool WIN>
 __device__ __forceinline__ void stage_span(const StftArgs& a, float* xst, float* wst, float2* tw, const float* xb, int s,
                                            int span) {
     const int tid = threadIdx.x;
-    const float2 t = reinterpret_cast<const float2*>(kFftTable.v)[min(tid, kTwSlots - 1)];
+    const float2 t = reinterpret_cast<const float2*>(kFftTable.v)[min(tid, kTwFwd - 1)];
     float4 w = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if constexpr (WIN) w = ld4_any(a.w + 4 * tid);
     if (s >= 0 && s + span <= a.L) {
@@ -434,7 +441,7 @@ __device__ __forceinline__ void stage_span(const StftArgs& a, float* xst, float*
             }
         }
     }
-    if (tid < kTwSlots) tw[tid] = t;
+    if (tid < kTwFwd) tw[tid] = t;
     if constexpr (WIN)
         *reinterpret_cast<float4*>(wst + 4 * tid) = make_float4(w.x * a.scale, w.y * a.scale, w.z * a.scale, w.w * a.scale);
 }
@@ -446,7 +453,7 @@ __device__ __forceinline__ void stage_span(const StftArgs& a, float* xst, float*
 // conflicts: 25.5 us.  Half slots, per-lane twiddle tables and layouts without conflicts: 21.4.
 // The same with layouts padded by p/16, whose 32-bit reads conflict: 28.4.
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(MBRT_STFT_WPE))) void stft_kernel(StftArgs a) {
-    __shared__ __attribute__((aligned(16))) float lds[kTF * kSlot + 2 * kTwSlots];
+    __shared__ __attribute__((aligned(16))) float lds[kTF * kSlot + 2 * kTwFwd];
     float2* tw = reinterpret_cast<float2*>(lds + kTF * kSlot);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     // workgroup = frames t0 .. t0 + nf - 1 of signal b: one of the first `whole` groups of kTF frames,
@@ -495,7 +502,7 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(MBRT_STFT_W
         }
         __syncthreads();  // the staging area becomes the frame slots
     } else {
-        if (threadIdx.x < kTwSlots) tw[threadIdx.x] = reinterpret_cast<const float2*>(kFftTable.v)[threadIdx.x];
+        if (threadIdx.x < kTwFwd) tw[threadIdx.x] = reinterpret_cast<const float2*>(kFftTable.v)[threadIdx.x];
         if (live) {
             load_frame(a, xb, s + wave * a.hop, lane, v);
 #pragma unroll
@@ -674,7 +681,8 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(MBRT_ISTFT_
         }
         mid = gld<MBRT_NT_STFT & 1>(src + (int64_t)512 * a.T);
     }
-    const float2 t = reinterpret_cast<const float2*>(kFftTable.v)[min((int)threadIdx.x, kTwSlots - 1)];
+    const float2* table = reinterpret_cast<const float2*>(kFftTable.v);
+    const float2 tlo = table[threadIdx.x], thi = table[min((int)threadIdx.x + kNT, kTwSlots - 1)];
     // The spectra enter through LDS: X[k], k <= 512, at place k of the frame's slot and
     // X[1024 - k] kHi further.  Places are rotated by the frame (p ^ 2 frame within 16), so that
     // the 8 frames x 2 bins that 16 lanes write at a time fall on different banks.
@@ -692,55 +700,27 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(MBRT_ISTFT_
         st[512 + rt] = bin_f32(mid);
         st[kHi + 512 + rt] = bin_f32(mid);
     }
-    if (threadIdx.x < kTwSlots) tw[threadIdx.x] = t;
+    tw[threadIdx.x] = tlo;
+    if (threadIdx.x + kNT < kTwSlots) tw[threadIdx.x + kNT] = thi;
     __syncthreads();
     // Each lane forms the 16 bins of its first radix-16 pass, Z[l + 64 a]: for a < 8 from pair
-    // k = l + 64 a, for a = 15 - h as the mirror of pair k = m + 64 h, m = 64 - l.  Their twiddles
-    // W^-k have the angles a pi / 16 + th and (h + 1) pi / 16 - th, th that of S[l]; those
-    // past pi / 4 are swaps of the others.
+    // k = l + 64 a, for a = 15 - h as the mirror of pair k = m + 64 h, m = 64 - l.  The twiddles W^-k
+    // of k and 512 - k have each other's cosine and sine, so eight reads serve all sixteen.
     float* slot = lds + wave * kSlotInv;
     cf zA[4], zB[4], zC[4], zD[4];
     if (live) {
         const float2* xk = reinterpret_cast<const float2*>(slot);
-        constexpr float Kc[4] = {1.0f, 0.98078528040323044913f, 0.92387953251128675613f, 0.83146961230254523708f};
-        constexpr float Ks[4] = {0.0f, 0.19509032201612826785f, 0.38268343236508977173f, 0.55557023301960222474f};
-        constexpr float K4 = 0.70710678118654752440f;  // cos, sin of a pi / 16, a < 4, and pi / 4
         const int rw = wave << 1, p = lane ^ rw, m = (64 - lane) ^ rw;
-        const cf w = lds_ld(tw, kTwS + lane);
-        const float c = w.x, n = -w.y;
+        const float2 *tp = tw + kTwS + lane, *tm = tw + kTwS - lane;
         cf v[16];
 #pragma unroll
-        for (int a = 0; a < 8; ++a) {
-            float cp, sp;  // a pi / 16 + th
-            if (a < 4) {
-                cp = a ? Kc[a] * c - Ks[a] * n : c;
-                sp = a ? Ks[a] * c + Kc[a] * n : n;
-            } else if (a == 4) {
-                cp = K4 * (c - n);
-                sp = K4 * (c + n);
-            } else {
-                cp = Ks[8 - a] * c - Kc[8 - a] * n;
-                sp = Kc[8 - a] * c + Ks[8 - a] * n;
-            }
-            v[a] = c2r_bin<false>(xk[p + 64 * a], xk[kHi + p + 64 * a], cp, sp);
-        }
-#pragma unroll
-        for (int a = 1; a <= 8; ++a) {
-            float cm, sm;  // a pi / 16 - th
-            if (a < 4) {
-                cm = Kc[a] * c + Ks[a] * n;
-                sm = Ks[a] * c - Kc[a] * n;
-            } else if (a == 4) {
-                cm = K4 * (c + n);
-                sm = K4 * (c - n);
-            } else if (a < 8) {
-                cm = Ks[8 - a] * c + Kc[8 - a] * n;
-                sm = Kc[8 - a] * c - Ks[8 - a] * n;
-            } else {
-                cm = n;
-                sm = c;
-            }
-            v[16 - a] = c2r_bin<true>(xk[m + 64 * (a - 1)], xk[kHi + m + 64 * (a - 1)], cm, sm);
+        for (int a = 0; a < 4; ++a) {  // k = l + 64 a and 512 - k, and k = 64 (a + 1) - l and 512 - k
+            const cf w = lds_ld(tp, 64 * a), u = lds_ld(tm, 64 * (a + 1));
+            const int a7 = 7 - a;
+            v[a] = c2r_bin<false>(xk[p + 64 * a], xk[kHi + p + 64 * a], w.x, -w.y);
+            v[8 + a] = c2r_bin<true>(xk[m + 64 * a7], xk[kHi + m + 64 * a7], -w.y, w.x);
+            v[a7] = c2r_bin<false>(xk[p + 64 * a7], xk[kHi + p + 64 * a7], -u.y, u.x);
+            v[15 - a] = c2r_bin<true>(xk[m + 64 * a], xk[kHi + m + 64 * a], u.x, -u.y);
         }
         fft1024<true>(v, slot, tw, lane, zA, zB, zC, zD);
     }
