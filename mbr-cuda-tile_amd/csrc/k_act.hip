@@ -186,11 +186,12 @@ struct GateArgs {
     FastDiv n_div;     // N
     FastDiv sb_div;    // MBRT_GATE_TPW * groups per token
     int tpw_ok;        // B * N is a multiple of MBRT_GATE_TPW
-    int cold;          // the attention values are too large to be cached
     int fb;            // bf16 intermediates (element kernel; the vector kernel takes FB)
 };
 
-template <int ADT, int GDT, int ODT, bool FB>
+// HOT: the attention values are small enough to be cached, so ordinary loads; an instance, as in
+// the qkv split.
+template <int ADT, int GDT, int ODT, bool FB, bool HOT>
 __global__ __launch_bounds__(kThreads) void gate_merge_vec_kernel(GateArgs a) {
     constexpr int VE = (ADT == F32 || ODT == F32) ? 4 : 8;
     // chunks of kThreads * kUGate groups; a grid smaller than the chunk count walks them
@@ -233,10 +234,8 @@ __global__ __launch_bounds__(kThreads) void gate_merge_vec_kernel(GateArgs a) {
         srcs[u] = src;
         gl[u] = ld1<GDT>(a.gate, (int64_t)token * a.H + h);
     }
-    load_by<MBRT_NT_GATE>(a.cold, [&](auto nt) {
 #pragma unroll
-        for (int u = 0; u < kUGate; ++u) av[u].template load<decltype(nt)::value>(a.attn, srcs[u]);
-    });
+    for (int u = 0; u < kUGate; ++u) av[u].template load<HOT ? MBRT_NT_GATE & 2 : MBRT_NT_GATE>(a.attn, srcs[u]);
 #pragma unroll
     for (int u = 0; u < kUGate; ++u) {
         const int64_t g = base + u * kThreads;
@@ -426,20 +425,27 @@ int mbrt_sigmoid_gate_merge(const void* attn, int attn_dtype, const void* gate, 
         a.n_div = make_fastdiv((uint32_t)N);
         a.sb_div = make_fastdiv((uint32_t)(MBRT_GATE_TPW * H * D / ve));
         a.tpw_ok = (B * N) % MBRT_GATE_TPW == 0 ? 1 : 0;
-        a.cold = cold_input(total * dt_size(attn_dtype));
+        const bool cold = cold_input(total * dt_size(attn_dtype), MBRT_HOT_BYTES_GATE);
         with_dt(attn_dtype, [&](auto at) {
             with_dt(gate_dtype, [&](auto gt) {
                 with_dt(out_dtype, [&](auto ot) {
                     constexpr int A = decltype(at)::value, G = decltype(gt)::value, O = decltype(ot)::value;
                     dim3 grid = vec_grid(a.groups, kUGate);
                     if (MBRT_GATE_BPC > 0) grid.x = (unsigned)std::min<int64_t>(grid.x, (int64_t)cu_count() * MBRT_GATE_BPC);
+                    auto launch = [&](auto fb) {
+                        constexpr bool FB = decltype(fb)::value;
+                        if (cold)
+                            hipLaunchKernelGGL((gate_merge_vec_kernel<A, G, O, FB, false>), grid, dim3(kThreads), 0, st, a);
+                        else
+                            hipLaunchKernelGGL((gate_merge_vec_kernel<A, G, O, FB, true>), grid, dim3(kThreads), 0, st, a);
+                    };
                     if constexpr (A == BF16) {
                         if (a.fb) {
-                            hipLaunchKernelGGL((gate_merge_vec_kernel<A, G, O, true>), grid, dim3(kThreads), 0, st, a);
+                            launch(std::true_type());
                             return;
                         }
                     }
-                    hipLaunchKernelGGL((gate_merge_vec_kernel<A, G, O, false>), grid, dim3(kThreads), 0, st, a);
+                    launch(std::false_type());
                 });
             });
         });

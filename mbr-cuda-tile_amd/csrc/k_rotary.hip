@@ -116,12 +116,13 @@ struct SplitArgs {
     const void* sinp;
     int64_t B, N, H, D, outN;
     int fb;  // bf16 intermediates (scalar kernel; the vector kernel takes FB)
-    int cold;  // qkv is too large to be cached
 };
 
 // One thread per VE-element group of the [B, H, outN, D] outputs (q, k and v together);
-// the three qkv loads and the table loads are issued before any use.
-template <int IDT, int ODT, int TDT, bool FB>
+// the three qkv loads and the table loads are issued before any use.  HOT: qkv is small enough to
+// be cached, so ordinary loads; an instance, because a run-time choice here and in the gate merge
+// cost the large calls 1 % (the steps of [801, 60] rows 101.9 -> 102.8 us).
+template <int IDT, int ODT, int TDT, bool FB, bool HOT>
 __global__ __launch_bounds__(kThreads) void split_qkv_vec_kernel(SplitArgs a, uint32_t groups, FastDiv gpr,
                                                           FastDiv outn_div, FastDiv h_div) {
     constexpr int VE = (IDT == F32 || ODT == F32) ? 4 : 8;
@@ -138,12 +139,10 @@ __global__ __launch_bounds__(kThreads) void split_qkv_vec_kernel(SplitArgs a, ui
     const int64_t t = nn * (a.D / 2) + (int64_t)c * (VE / 2);
     Vec<IDT, VE> vq, vk, vv;
     Vec<TDT, VE / 2> cv, sv;
-    load_by<MBRT_NT_ROT>(a.cold, [&](auto nt) {
-        constexpr int NT = decltype(nt)::value;
-        vq.template load<NT>(a.qkv, src);
-        vk.template load<NT>(a.qkv, src + a.H * a.D);
-        vv.template load<NT>(a.qkv, src + 2 * a.H * a.D);
-    });
+    constexpr int NT = HOT ? MBRT_NT_ROT & 2 : MBRT_NT_ROT;
+    vq.template load<NT>(a.qkv, src);
+    vk.template load<NT>(a.qkv, src + a.H * a.D);
+    vv.template load<NT>(a.qkv, src + 2 * a.H * a.D);
     cv.load(a.cosp, t);
     sv.load(a.sinp, t);
     float xq[VE], xk[VE], xv[VE], cs[VE / 2], sn[VE / 2];
@@ -326,25 +325,30 @@ int mbrt_split_qkv_heads_rotary(const void* qkv, int qkv_dtype, const void* cos_
                      tab_al && groups < (1ll << 31);
     if (vec) {
         const dim3 grid((unsigned)ceil_div(groups, kThreads));
-        a.cold = cold_input(3 * B * N * H * D * dt_size(qkv_dtype));
+        const bool cold = cold_input(3 * B * N * H * D * dt_size(qkv_dtype));
         const FastDiv gpr = make_fastdiv((uint32_t)(D / ve)), od = make_fastdiv((uint32_t)out_N),
                       hd = make_fastdiv((uint32_t)H);
         with_dt(qkv_dtype, [&](auto it) {
             with_dt(out_dtype, [&](auto ot) {
                 constexpr int IDTv = decltype(it)::value, ODTv = decltype(ot)::value;
+                auto launch = [&](auto tt, auto fb) {
+                    constexpr int TDTv = decltype(tt)::value;
+                    constexpr bool FB = decltype(fb)::value;
+                    if (cold)
+                        hipLaunchKernelGGL((split_qkv_vec_kernel<IDTv, ODTv, TDTv, FB, false>), grid, dim3(kThreads), 0,
+                                           st, a, (uint32_t)groups, gpr, od, hd);
+                    else
+                        hipLaunchKernelGGL((split_qkv_vec_kernel<IDTv, ODTv, TDTv, FB, true>), grid, dim3(kThreads), 0,
+                                           st, a, (uint32_t)groups, gpr, od, hd);
+                };
                 if constexpr (IDTv == BF16 && ODTv == BF16) {
                     if (a.fb && trig_dtype == F32) {
-                        hipLaunchKernelGGL((split_qkv_vec_kernel<IDTv, ODTv, F32, true>), grid, dim3(kThreads), 0, st,
-                                           a, (uint32_t)groups, gpr, od, hd);
+                        launch(std::integral_constant<int, F32>(), std::true_type());
                         return;
                     }
                 }
-                if (trig_dtype == F32)
-                    hipLaunchKernelGGL((split_qkv_vec_kernel<IDTv, ODTv, F32, false>), grid, dim3(kThreads), 0, st, a,
-                                       (uint32_t)groups, gpr, od, hd);
-                else
-                    hipLaunchKernelGGL((split_qkv_vec_kernel<IDTv, ODTv, BF16, false>), grid, dim3(kThreads), 0, st, a,
-                                       (uint32_t)groups, gpr, od, hd);
+                if (trig_dtype == F32) launch(std::integral_constant<int, F32>(), std::false_type());
+                else launch(std::integral_constant<int, BF16>(), std::false_type());
             });
         });
     } else {

@@ -17,9 +17,14 @@
 // inputs gain as much while they are warm (split of 37 MB 14.5 -> 12.1), but in a chain of calls they
 // are cold by then and lose: the token step of 401 frames 61.6 -> 62.9 us with 40 MB as the limit.
 // RMSNorm and GLU, whose second operands come from further back, take MBRT_HOT_BYTES_ACT:
-// with 20 MB the token step of 201 frames ran 33.9 -> 34.9 us over three buffer sets.
+// with 20 MB the token step of 201 frames ran 33.9 -> 34.9 us over three buffer sets.  The gate merge
+// takes MBRT_HOT_BYTES_GATE: in the frequency attention's chain of calls, 12.3 MB into it ([200, 60]
+// rows) ran 31.8 us with ordinary loads and 31.2 without, 18.4 MB 44.8 and 44.0.
 #ifndef MBRT_HOT_BYTES
 #define MBRT_HOT_BYTES (20ll << 20)
+#endif
+#ifndef MBRT_HOT_BYTES_GATE
+#define MBRT_HOT_BYTES_GATE (8ll << 20)
 #endif
 #ifndef MBRT_HOT_BYTES_ACT
 #define MBRT_HOT_BYTES_ACT (12ll << 20)
