@@ -200,7 +200,7 @@ __global__ __launch_bounds__(kThreads) void gate_merge_vec_kernel(GateArgs a) {
     const int64_t base = chunk * (kThreads * kUGate) + threadIdx.x;
     Vec<ADT, VE> av[kUGate];
     float gl[kUGate];
-    int64_t dst[kUGate], srcs[kUGate];
+    int64_t dst[kUGate];
 #pragma unroll
     for (int u = 0; u < kUGate; ++u) {
         const uint32_t g = (uint32_t)clamp_group(base + u * kThreads, a.groups);
@@ -231,11 +231,9 @@ __global__ __launch_bounds__(kThreads) void gate_merge_vec_kernel(GateArgs a) {
             }
             dst[u] = (int64_t)g * VE;
         }
-        srcs[u] = src;
+        av[u].template load<HOT ? MBRT_NT_GATE & 2 : MBRT_NT_GATE>(a.attn, src);
         gl[u] = ld1<GDT>(a.gate, (int64_t)token * a.H + h);
     }
-#pragma unroll
-    for (int u = 0; u < kUGate; ++u) av[u].template load<HOT ? MBRT_NT_GATE & 2 : MBRT_NT_GATE>(a.attn, srcs[u]);
 #pragma unroll
     for (int u = 0; u < kUGate; ++u) {
         const int64_t g = base + u * kThreads;

@@ -19,7 +19,7 @@
 // RMSNorm and GLU, whose second operands come from further back, take MBRT_HOT_BYTES_ACT:
 // with 20 MB the token step of 201 frames ran 33.9 -> 34.9 us over three buffer sets.  The gate merge
 // takes MBRT_HOT_BYTES_GATE: in the frequency attention's chain of calls, 12.3 MB into it ([200, 60]
-// rows) ran 31.8 us with ordinary loads and 31.2 without, 18.4 MB 44.8 and 44.0.
+// rows) ran 31.8 us with ordinary loads and 31.2 without, 18.4 MB 44.8 and 43.2.
 #ifndef MBRT_HOT_BYTES
 #define MBRT_HOT_BYTES (20ll << 20)
 #endif
