@@ -125,9 +125,26 @@ def _objects(srcdir: Path, names: list[str], tag: str, build_dir: Path, defines:
     return objs
 
 
+def _torch_dir() -> Path | None:
+    spec = importlib.util.find_spec("torch")
+    return Path(spec.submodule_search_locations[0]) if spec is not None and spec.submodule_search_locations else None
+
+
+def _calls_lack() -> str | None:
+    """What the binding's extension module needs and this Python lacks, or None."""
+    torch_dir = _torch_dir()
+    if torch_dir is None:
+        return "torch"
+    if not (torch_dir / "include" / "c10" / "hip" / "HIPStream.h").exists():
+        return "torch's ROCm headers"
+    if not (Path(sysconfig.get_paths()["include"]) / "Python.h").exists():
+        return "Python's headers"
+    return None
+
+
 def _compile_calls(build_dir: Path, verbose: bool) -> Path:
     """The binding's extension module: host code against torch's and Python's headers."""
-    torch_dir = Path(importlib.util.find_spec("torch").submodule_search_locations[0])
+    torch_dir = _torch_dir()
     obj = build_dir / "p_calls.o"
     _run([HIPCC, "-x", "c++", "-O2", "-fPIC", "-fvisibility=hidden", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1",
           "-DUSE_ROCM", f"-I{REPO / 'include'}", "-isystem", str(torch_dir / "include"), "-isystem",
@@ -139,10 +156,9 @@ def _compile_calls(build_dir: Path, verbose: bool) -> Path:
 
 def _link_calls(obj: Path, lib_dir: Path, verbose: bool) -> Path:
     """torch's libraries are loaded before the module is, by the package's `import torch`."""
-    torch_lib = Path(importlib.util.find_spec("torch").submodule_search_locations[0]) / "lib"
     ext = lib_dir / "_mbrt_calls.so"
     tmp = ext.with_suffix(".so.tmp")
-    _run([HIPCC, "-shared", "-fPIC", "-o", str(tmp), str(obj), f"-L{lib_dir}", "-lmbrt", f"-L{torch_lib}",
+    _run([HIPCC, "-shared", "-fPIC", "-o", str(tmp), str(obj), f"-L{lib_dir}", "-lmbrt", f"-L{_torch_dir() / 'lib'}",
           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"], verbose)
     os.replace(tmp, ext)
     return ext
@@ -150,30 +166,37 @@ def _link_calls(obj: Path, lib_dir: Path, verbose: bool) -> Path:
 
 def build(jobs: int | None = None, verbose: bool = False, defines: list[str] | None = None,
           out_dir: Path | str | None = None) -> dict[str, Path]:
-    """Compile every source and link the libraries and the extension module; returns their paths."""
+    """Compile every source, link the two libraries and then the binding's extension module (left
+    out, with a message, where torch or a header that it needs is missing: the libraries need
+    neither); returns their paths."""
     jobs = jobs or min(8, os.cpu_count() or 4)
     defines = list(defines or [])
     lib_dir = Path(out_dir) if out_dir else LIB
     build_dir = lib_dir / "_build" if out_dir else BUILD
     lib_dir.mkdir(parents=True, exist_ok=True)
     build_dir.mkdir(parents=True, exist_ok=True)
+    lack = _calls_lack()
     with cf.ThreadPoolExecutor(max_workers=1) as ex:
-        calls_obj = ex.submit(_compile_calls, build_dir, verbose)  # beside the kernels
+        calls_obj = None if lack else ex.submit(_compile_calls, build_dir, verbose)  # beside the kernels
         kobjs = _objects(CSRC, KERNEL_SOURCES, "k", build_dir, defines, jobs, verbose)
-    libmbrt = lib_dir / "libmbrt.so"
-    tmp = libmbrt.with_suffix(".so.tmp")
-    _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, kobjs)], verbose)
-    os.replace(tmp, libmbrt)
-    out = {"libmbrt": libmbrt, "mbrt_calls": _link_calls(calls_obj.result(), lib_dir, verbose)}
-    tsrc = [n for n in TENSOR_SOURCES if (HOST / n).exists()]
-    if tsrc:
-        tobjs = _objects(HOST, tsrc, "t", build_dir, defines, jobs, verbose)
-        libt = lib_dir / "libmbrt_tensor.so"
-        tmp = libt.with_suffix(".so.tmp")
-        _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, tobjs),
-              f"-L{lib_dir}", "-lmbrt", "-Wl,-rpath,$ORIGIN"], verbose)
-        os.replace(tmp, libt)
-        out["libmbrt_tensor"] = libt
+        libmbrt = lib_dir / "libmbrt.so"
+        tmp = libmbrt.with_suffix(".so.tmp")
+        _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, kobjs)], verbose)
+        os.replace(tmp, libmbrt)
+        out = {"libmbrt": libmbrt}
+        tsrc = [n for n in TENSOR_SOURCES if (HOST / n).exists()]
+        if tsrc:
+            tobjs = _objects(HOST, tsrc, "t", build_dir, defines, jobs, verbose)
+            libt = lib_dir / "libmbrt_tensor.so"
+            tmp = libt.with_suffix(".so.tmp")
+            _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, tobjs),
+                  f"-L{lib_dir}", "-lmbrt", "-Wl,-rpath,$ORIGIN"], verbose)
+            os.replace(tmp, libt)
+            out["libmbrt_tensor"] = libt
+    if lack:
+        print(f"mbrt: the Python binding's native calls are not built: {lack} not found for {sys.executable}", flush=True)
+    else:
+        out["mbrt_calls"] = _link_calls(calls_obj.result(), lib_dir, verbose)
     return out
 
 

@@ -1,0 +1,52 @@
+"""CPU checks of the build script: what it links, and in which order, when a part is missing.
+The compiler is stood in for by a function that records its output files."""
+from __future__ import annotations
+
+import importlib.util
+from pathlib import Path
+
+import pytest
+
+PKG = Path(__file__).resolve().parent.parent / "mbr-cuda-tile_amd"
+
+
+@pytest.fixture
+def pkg_build(monkeypatch):
+    spec = importlib.util.spec_from_file_location("mbrt_build_under_test", PKG / "build.py")
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+
+    def run(cmd, verbose):
+        if any(c.endswith(mod.fail) for c in cmd if mod.fail):
+            raise RuntimeError("command failed")
+        Path(cmd[cmd.index("-o") + 1]).touch()
+
+    mod.fail = ""
+    monkeypatch.setattr(mod, "_run", run)
+    return mod
+
+
+def test_build_links_everything(pkg_build, tmp_path):
+    out = pkg_build.build(out_dir=tmp_path)
+    assert set(out) == {"libmbrt", "libmbrt_tensor", "mbrt_calls"} and all(p.exists() for p in out.values())
+
+
+def test_build_without_torch_links_the_libraries(pkg_build, tmp_path, monkeypatch, capsys):
+    find = importlib.util.find_spec
+    monkeypatch.setattr(importlib.util, "find_spec", lambda n, *a: None if n == "torch" else find(n, *a))
+    out = pkg_build.build(out_dir=tmp_path)
+    assert set(out) == {"libmbrt", "libmbrt_tensor"} and all(p.exists() for p in out.values())
+    assert "native calls are not built: torch not found" in capsys.readouterr().out
+
+
+def test_build_without_python_headers_links_the_libraries(pkg_build, tmp_path, monkeypatch, capsys):
+    monkeypatch.setattr(pkg_build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    assert set(pkg_build.build(out_dir=tmp_path)) == {"libmbrt", "libmbrt_tensor"}
+    assert "Python's headers not found" in capsys.readouterr().out
+
+
+def test_build_error_in_the_extension_comes_after_the_libraries(pkg_build, tmp_path):
+    pkg_build.fail = "calls.cpp"
+    with pytest.raises(RuntimeError, match="command failed"):
+        pkg_build.build(out_dir=tmp_path)
+    assert (tmp_path / "libmbrt.so").exists() and (tmp_path / "libmbrt_tensor.so").exists()
