@@ -3,7 +3,8 @@
 Outputs (git-ignored, shipped with the source tree):
   mbr-cuda-tile_amd/lib/libmbrt.so        C-ABI + HIP kernels (include/mbrt.h)
   mbr-cuda-tile_amd/lib/libmbrt_tensor.so C++ Tensor / tensor_tile:: / mbr_tile:: layer
-  mbr-cuda-tile_amd/lib/_mbrt_calls.so    native calls of the Python binding (pyext/)
+  mbr-cuda-tile_amd/lib/_mbrt_calls.*.so  native calls of the Python binding (pyext/), for the
+                                          Python that runs this and its torch
 
 Usage: python mbr-cuda-tile_amd/build.py [-j N] [-v] [-D NAME=VALUE ...] [--out DIR]
 
@@ -17,6 +18,7 @@ import argparse
 import concurrent.futures as cf
 import importlib.util
 import os
+import runpy
 import shlex
 import subprocess
 import sys
@@ -156,7 +158,8 @@ def _compile_calls(build_dir: Path, verbose: bool) -> Path:
 
 def _link_calls(obj: Path, lib_dir: Path, verbose: bool) -> Path:
     """torch's libraries are loaded before the module is, by the package's `import torch`."""
-    ext = lib_dir / "_mbrt_calls.so"
+    version = runpy.run_path(str(_torch_dir() / "version.py"))["__version__"]
+    ext = lib_dir / f"_mbrt_calls.{sys.implementation.cache_tag}-torch{version}.so"
     tmp = ext.with_suffix(".so.tmp")
     _run([HIPCC, "-shared", "-fPIC", "-o", str(tmp), str(obj), f"-L{lib_dir}", "-lmbrt", f"-L{_torch_dir() / 'lib'}",
           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"], verbose)

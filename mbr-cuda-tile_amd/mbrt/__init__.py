@@ -2,12 +2,14 @@
 
 torch provides device memory and the stream only; every computation is a call into
 lib/libmbrt.so.  Each function enqueues on torch's current HIP stream (or `stream`).  The
-calls a model makes many times per chunk go through lib/_mbrt_calls.so (pyext/calls.cpp),
-which reads the tensors natively; the others through ctypes.
+calls a model makes many times per chunk go through an extension module built for this Python
+and torch (pyext/calls.cpp), which reads the tensors natively; the others, and all where that
+module is missing, through ctypes.
 """
 from __future__ import annotations
 
 import ctypes as C
+import warnings
 from typing import Sequence
 
 import torch
@@ -50,12 +52,26 @@ def _contig(*ts: torch.Tensor) -> None:
             raise ValueError("mbrt: expected a contiguous tensor")
 
 
+def _load_native():
+    """The native calls, or the same ones through ctypes where the module built is for another
+    Python or torch (or none is)."""
+    path = _abi.calls_path(torch.__version__)
+    lib()  # raises where nothing is built
+    if path.exists():
+        return _abi.load_calls(path)
+    warnings.warn(f"mbrt: {path.name} is not built (run python mbr-cuda-tile_amd/build.py with this Python): "
+                  "calls go through ctypes, at about 5 us more each", RuntimeWarning, stacklevel=4)
+    from . import _calls
+
+    return _calls
+
+
 class _Native:
     """Stands for the native calls until the first one, then loads them in its place."""
 
     def __getattr__(self, name):
         global _n
-        _n = _abi.load_calls()
+        _n = _load_native()
         return getattr(_n, name)
 
 

@@ -7,11 +7,11 @@ from __future__ import annotations
 
 import ctypes as C
 import importlib.util
+import sys
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent.parent
 LIB_PATH = PKG_DIR / "lib" / "libmbrt.so"
-CALLS_PATH = PKG_DIR / "lib" / "_mbrt_calls.so"
 
 MAX_DIMS = 8
 
@@ -155,11 +155,15 @@ def lib() -> C.CDLL:
     return _LIB
 
 
-def load_calls(path: Path | str = CALLS_PATH):
-    """The extension module of native calls (pyext/calls.cpp); it links libmbrt.so."""
-    path = Path(path)
-    if not path.exists():
-        raise ImportError(f"mbrt: {path} is not built (run python mbr-cuda-tile_amd/build.py)")
+def calls_path(torch_version: str) -> Path:
+    """The extension module of native calls (pyext/calls.cpp) for this Python and a torch version.  Both
+    are in its name, as by build.py: it is compiled against their headers, and loading it into
+    others is not safe."""
+    return PKG_DIR / "lib" / f"_mbrt_calls.{sys.implementation.cache_tag}-torch{torch_version}.so"
+
+
+def load_calls(path: Path):
+    """That module; it links libmbrt.so."""
     spec = importlib.util.spec_from_file_location("_mbrt_calls", path)
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)

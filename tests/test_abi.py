@@ -262,3 +262,35 @@ def test_native_calls_refuse_what_the_binding_documents(lib):
     assert mbrt.fill_(torch.empty(0), 1.0, stream=0).numel() == 0  # nothing to do: no launch
     with pytest.raises(mbrt.MbrtError, match="SHAPE"):
         mbrt.chunk_accumulate(x, x[0], y, y[0], 5, stream=0)
+
+
+def test_calls_without_the_extension_module(lib, monkeypatch, tmp_path):
+    """For a Python or torch that the extension module was not built for, the same calls go through
+    ctypes: the same functions, with the same refusals (the test above, over them)."""
+    import torch
+
+    import mbrt
+    from mbrt import _abi, _calls
+
+    native = _abi.load_calls(_abi.calls_path(torch.__version__))
+    names = {n for n in vars(native) if not n.startswith("__")} - {"init"}
+    assert names == {n for n, f in vars(_calls).items() if callable(f) and not n.startswith("_")}
+
+    monkeypatch.setattr(_abi, "calls_path", lambda version: tmp_path / f"{version}.so")
+    monkeypatch.setattr(mbrt, "_n", mbrt._Native())
+    with pytest.warns(RuntimeWarning, match="not built"):
+        mbrt.fill_(torch.empty(0), 1.0, stream=0)
+    assert mbrt._n is _calls
+    test_native_calls_refuse_what_the_binding_documents(lib)
+
+
+def test_extension_module_is_named_by_python_and_torch(lib):
+    import sys
+
+    import torch
+
+    from mbrt import _abi
+
+    name = _abi.calls_path(torch.__version__).name
+    assert sys.implementation.cache_tag in name and torch.__version__ in name
+    assert _abi.calls_path(torch.__version__).exists() and not _abi.calls_path("0.0").exists()

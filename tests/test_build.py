@@ -29,6 +29,10 @@ def pkg_build(monkeypatch):
 def test_build_links_everything(pkg_build, tmp_path):
     out = pkg_build.build(out_dir=tmp_path)
     assert set(out) == {"libmbrt", "libmbrt_tensor", "mbrt_calls"} and all(p.exists() for p in out.values())
+    torch = pytest.importorskip("torch")
+    from mbrt import _abi
+
+    assert out["mbrt_calls"].name == _abi.calls_path(torch.__version__).name  # the name that is loaded
 
 
 def test_build_without_torch_links_the_libraries(pkg_build, tmp_path, monkeypatch, capsys):
