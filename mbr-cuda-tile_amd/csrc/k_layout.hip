@@ -728,8 +728,10 @@ void launch_cat(CatArgs& a, hipStream_t st) {
 }
 
 // The sources in launches of at most kCatSrcs when they lie in ascending order without
-// overlap (a concat's always do) and the grid and column indices fit 32 bits; false
-// otherwise, and nothing is launched: the caller copies them one after another.
+// overlap (a concat's always do), none of them lies in the output's memory (one that does may
+// hold what an earlier source is to write there: copied one after another, they are in order) and
+// the grid and column indices fit 32 bits; false otherwise, and nothing is launched: the caller
+// copies them one after another.
 bool try_cat(char* out, const mbrt_cat_src* srcs, int n, int64_t outer, int64_t total_cat_dim, int64_t inner_bytes,
              hipStream_t st) {
     const int64_t pitch = total_cat_dim * inner_bytes;
@@ -740,6 +742,8 @@ bool try_cat(char* out, const mbrt_cat_src* srcs, int n, int64_t outer, int64_t 
         if (srcs[i].dim_size * inner_bytes == 0) continue;
         if (srcs[i].dim_offset < end) return false;
         end = srcs[i].dim_offset + srcs[i].dim_size;
+        const char* p = static_cast<const char*>(srcs[i].ptr);
+        if (p < out + outer * pitch && out < p + outer * srcs[i].dim_size * inner_bytes) return false;
         bits |= reinterpret_cast<uintptr_t>(srcs[i].ptr) | (uintptr_t)(srcs[i].dim_size * inner_bytes) |
                 (uintptr_t)(srcs[i].dim_offset * inner_bytes);
         ++live;

@@ -176,6 +176,22 @@ def test_cat_one_launch(orc, dev, outer, sizes, inner, dt, shift):
     assert_bitexact(to_host(out, dt), np.concatenate(parts, axis=1), "cat")
 
 
+# a source that lies in the output: what an earlier source has written there is what a later one
+# copies, as by one copy after another; and a source already in its place
+@pytest.mark.parametrize("n", [5, 1000, 300000])
+def test_cat_source_in_the_output(orc, dev, n):
+    say(f"cat with a source in the output n={n}")
+    a = orc.randn((n,), seed=8)
+    out = torch.zeros(2 * n, device="cuda")
+    mbrt.cat([to_dev(a, F32), out[:n]], 0, out)
+    torch.cuda.synchronize()
+    assert_bitexact(to_host(out, F32), np.concatenate([a, a]), "second source is the first one's place")
+    b = orc.randn((n,), seed=9)
+    mbrt.cat([out[:n], to_dev(b, F32)], 0, out)
+    torch.cuda.synchronize()
+    assert_bitexact(to_host(out, F32), np.concatenate([a, b]), "first source in its place")
+
+
 # ---- element-wise ----------------------------------------------------------------------------
 
 @pytest.mark.parametrize("n", [0, 1, 7, 8, 1000, 4099])
