@@ -655,68 +655,80 @@ bool try_pad_rows(const PadArgs& p, int esize, hipStream_t st) {
 // Bound by launches where the sources are small: the 60 per-band tensors of a chunk
 // ([1, 801, 28..520] f32, 51 MB moved) took 60 row copies of 2-3 us on the GPU, each ~2.5 us to
 // enqueue; one launch takes 12.3-12.7 us (4.1 TB/s; a plain copy of 50 MB: 4.8).  A thread
-// keeps one vector column of the output and walks kCatU rows of it, so the column's source
-// is looked up once (binary search of the offsets in LDS), a wave writes up to 1 KB of
+// keeps one vector column of the sources and walks kCatU rows of it, so the column's source
+// is looked up once (binary search of the columns in LDS), a wave writes up to 1 KB of
 // consecutive output, and a source's rows are read whole.  2 or 8 rows per thread: 13.7-13.9
 // and 13.6-14.0 us against 13.4-13.8 for 4, with non-temporal loads; the sources have usually
 // just been written, so ordinary loads are kept: 12.3-12.7 (and 12.7-12.9 with ordinary
 // stores too).
+// Vectors are of 16 bytes at any even alignment: one word size for all sources, the largest that
+// every address, row and offset allows, moved all of them in 2-byte words for one odd view.
+// Two bf16 sources of 64 MB, one of them off by an element: 93 us by one copy each, 187 in 2-byte
+// words, 60 as now; eight of 16 MB 70, 196 and 47.
 constexpr int kCatSrcs = 64;
 constexpr int kCatU = 4;  // rows per thread, all loads in flight before the first store
 
 struct CatArgs {
     const char* src[kCatSrcs];
-    uint32_t off[kCatSrcs];  // first vector of the source in an output row, ascending
-    uint32_t run[kCatSrcs];  // vectors per source row
-    char* dst;
+    int64_t dst[kCatSrcs];   // byte offset of the source in an output row
+    int64_t run[kCatSrcs];   // bytes per source row
+    uint32_t col[kCatSrcs];  // first of the source's vector columns, ascending
+    char* out;
     int64_t dst_pitch;       // bytes between output rows
     int64_t outer;           // rows
-    uint32_t col0, cols;     // the vector columns [col0, col0 + cols) that the sources span
+    uint32_t cols;           // vector columns of all sources
     uint32_t col_blocks;     // blocks side by side over the columns
     int n;
     int tx_shift;            // log2 of the columns per block
 };
 
-template <int W>
+// Vectors of V bytes at addresses aligned to A.  With A < V (V = 16) a source row's last vector is
+// moved back to end at the row's end, as in row_copy_any_kernel; else every row holds whole vectors.
+template <int V, int A>
 __global__ __launch_bounds__(kThreads) void cat_kernel(CatArgs a) {
-    typedef typename WordOf<W>::T Word;
+    typedef typename WordOf<V>::T Word;
     __shared__ const char* src[kCatSrcs];
-    __shared__ uint32_t off[kCatSrcs], run[kCatSrcs];
+    __shared__ int64_t dst[kCatSrcs], run[kCatSrcs];
+    __shared__ uint32_t col[kCatSrcs];
     if ((int)threadIdx.x < a.n) {
         src[threadIdx.x] = a.src[threadIdx.x];
-        off[threadIdx.x] = a.off[threadIdx.x];
+        dst[threadIdx.x] = a.dst[threadIdx.x];
         run[threadIdx.x] = a.run[threadIdx.x];
+        col[threadIdx.x] = a.col[threadIdx.x];
     }
     __syncthreads();
     const uint32_t rb = blockIdx.x / a.col_blocks, cb = blockIdx.x - rb * a.col_blocks;
     const uint32_t tx = threadIdx.x & ((1u << a.tx_shift) - 1), ty = threadIdx.x >> a.tx_shift;
     const uint32_t ry = kThreads >> a.tx_shift;  // rows per step of the block
+    const bool live = (cb << a.tx_shift) + tx < a.cols;
     const uint32_t c = min((cb << a.tx_shift) + tx, a.cols - 1);
-    const uint32_t col = a.col0 + c;
     int s = 0;  // the last source that starts at or before the column
 #pragma unroll
     for (int step = kCatSrcs / 2; step > 0; step >>= 1)
-        if (s + step < a.n && off[s + step] <= col) s += step;
-    const uint32_t in = col - off[s], rv = run[s];
-    const bool live = (cb << a.tx_shift) + tx < a.cols && in < rv;  // not in a gap between sources
-    const char* sp = src[s] + (int64_t)min(in, rv - 1) * W;
-    const int64_t pitch = (int64_t)rv * W;
+        if (s + step < a.n && col[s + step] <= c) s += step;
+    const int64_t pitch = run[s];
+    int64_t in = (int64_t)(c - col[s]) * V;
+    if constexpr (A < V) in = min(in, pitch - V);
+    const char* sp = src[s] + in;
+    char* dp = a.out + dst[s] + in;
     const int64_t row0 = (int64_t)rb * (ry * kCatU) + ty;
     Word v[kCatU];
 #pragma unroll
     for (int u = 0; u < kCatU; ++u) {
-        const int64_t row = min(row0 + (int64_t)(u * ry), a.outer - 1);
-        v[u] = gld<MBRT_NT_CAT>(reinterpret_cast<const Word*>(sp + row * pitch));
+        const char* p = sp + min(row0 + (int64_t)(u * ry), a.outer - 1) * pitch;
+        if constexpr (A < V) v[u] = ld_any<MBRT_NT_CAT, A>(p);
+        else v[u] = gld<MBRT_NT_CAT>(reinterpret_cast<const Word*>(p));
     }
-    char* dp = a.dst + (int64_t)col * W;
 #pragma unroll
     for (int u = 0; u < kCatU; ++u) {
         const int64_t row = row0 + (int64_t)(u * ry);
-        if (live && row < a.outer) gst<MBRT_NT_CAT>(reinterpret_cast<Word*>(dp + row * a.dst_pitch), v[u]);
+        if (!live || row >= a.outer) continue;
+        if constexpr (A < V) st_any<MBRT_NT_CAT, A>(dp + row * a.dst_pitch, v[u]);
+        else gst<MBRT_NT_CAT>(reinterpret_cast<Word*>(dp + row * a.dst_pitch), v[u]);
     }
 }
 
-template <int W>
+template <int V, int A>
 void launch_cat(CatArgs& a, hipStream_t st) {
     int sh = 0;
     while ((1u << sh) < a.cols && (1 << sh) < kThreads) ++sh;
@@ -724,59 +736,67 @@ void launch_cat(CatArgs& a, hipStream_t st) {
     a.col_blocks = (uint32_t)ceil_div(a.cols, int64_t(1) << sh);
     const int64_t rows = (int64_t)(kThreads >> sh) * kCatU;
     const int64_t blocks = ceil_div(a.outer, rows) * a.col_blocks;
-    hipLaunchKernelGGL(cat_kernel<W>, dim3((unsigned)blocks), dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL((cat_kernel<V, A>), dim3((unsigned)blocks), dim3(kThreads), 0, st, a);
 }
 
 // The sources in launches of at most kCatSrcs when they lie in ascending order without
-// overlap (a concat's always do), none of them lies in the output's memory (one that does may
-// hold what an earlier source is to write there: copied one after another, they are in order) and
-// the grid and column indices fit 32 bits; false otherwise, and nothing is launched: the caller
+// overlap (a concat's always do), none of them lies in the output's memory (one that does may hold
+// what an earlier source is to write there: copied one after another, they are in order) and the
+// grid and column indices fit 32 bits; false otherwise, and nothing is launched: the caller
 // copies them one after another.
 bool try_cat(char* out, const mbrt_cat_src* srcs, int n, int64_t outer, int64_t total_cat_dim, int64_t inner_bytes,
              hipStream_t st) {
     const int64_t pitch = total_cat_dim * inner_bytes;
     uintptr_t bits = reinterpret_cast<uintptr_t>(out) | (uintptr_t)pitch;
-    int64_t end = 0;
-    int live = 0;
+    int64_t end = 0, used = 0, shortest = pitch, live = 0;
     for (int i = 0; i < n; ++i) {
-        if (srcs[i].dim_size * inner_bytes == 0) continue;
+        const int64_t run = srcs[i].dim_size * inner_bytes;
+        if (run == 0) continue;
         if (srcs[i].dim_offset < end) return false;
         end = srcs[i].dim_offset + srcs[i].dim_size;
         const char* p = static_cast<const char*>(srcs[i].ptr);
-        if (p < out + outer * pitch && out < p + outer * srcs[i].dim_size * inner_bytes) return false;
-        bits |= reinterpret_cast<uintptr_t>(srcs[i].ptr) | (uintptr_t)(srcs[i].dim_size * inner_bytes) |
-                (uintptr_t)(srcs[i].dim_offset * inner_bytes);
+        if (p < out + outer * pitch && out < p + outer * run) return false;
+        bits |= reinterpret_cast<uintptr_t>(p) | (uintptr_t)run | (uintptr_t)(srcs[i].dim_offset * inner_bytes);
+        used += run;
+        shortest = std::min(shortest, run);
         ++live;
     }
     if (live < 2) return false;
-    const int W = (bits & 15) == 0 ? 16 : (bits & 7) == 0 ? 8 : (bits & 3) == 0 ? 4 : (bits & 1) == 0 ? 2 : 1;
+    // long rows of large sources: a launch apiece costs little
+    if (used / live >= MBRT_CAT_ROW && used * outer >= std::max(live * MBRT_CAT_SRC, MBRT_CAT_ALL)) return false;
+    // the alignment that all addresses, rows and offsets have; 16-byte vectors at any even one where
+    // every row holds one
+    const int A = (bits & 15) == 0 ? 16 : (bits & 7) == 0 ? 8 : (bits & 3) == 0 ? 4 : (bits & 1) == 0 ? 2 : 1;
+    const int V = A > 1 && shortest >= 16 ? 16 : A;
+    const int64_t most = pitch / V + live;  // columns
     // blocks <= (outer / kCatU + 1) * (columns / kThreads + 1), kept below the grid limit
-    if (pitch / W >= (int64_t(1) << 31) || outer >= (int64_t(1) << 32) ||
-        (outer / kCatU + 1) * (pitch / W / kThreads + 1) > kMaxGridX)
+    if (most >= (int64_t(1) << 31) || outer >= (int64_t(1) << 32) ||
+        (outer / kCatU + 1) * (most / kThreads + 1) > kMaxGridX)
         return false;
     CatArgs a{};
-    a.dst = out;
+    a.out = out;
     a.dst_pitch = pitch;
     a.outer = outer;
     for (int i = 0; i < n; ++i) {
         const int64_t run = srcs[i].dim_size * inner_bytes;
         if (run == 0) continue;
         a.src[a.n] = static_cast<const char*>(srcs[i].ptr);
-        a.off[a.n] = (uint32_t)(srcs[i].dim_offset * inner_bytes / W);
-        a.run[a.n] = (uint32_t)(run / W);
+        a.dst[a.n] = srcs[i].dim_offset * inner_bytes;
+        a.run[a.n] = run;
+        a.col[a.n] = a.cols;
+        a.cols += (uint32_t)ceil_div(run, V);
         ++a.n;
         --live;
         if (a.n < kCatSrcs && live > 0) continue;
-        a.col0 = a.off[0];
-        a.cols = a.off[a.n - 1] + a.run[a.n - 1] - a.off[0];
-        switch (W) {
-            case 16: launch_cat<16>(a, st); break;
-            case 8: launch_cat<8>(a, st); break;
-            case 4: launch_cat<4>(a, st); break;
-            case 2: launch_cat<2>(a, st); break;
-            default: launch_cat<1>(a, st); break;
-        }
+        if (V == 16 && A == 16) launch_cat<16, 16>(a, st);
+        else if (V == 16 && A >= 4) launch_cat<16, 4>(a, st);
+        else if (V == 16) launch_cat<16, 2>(a, st);
+        else if (V == 8) launch_cat<8, 8>(a, st);
+        else if (V == 4) launch_cat<4, 4>(a, st);
+        else if (V == 2) launch_cat<2, 2>(a, st);
+        else launch_cat<1, 1>(a, st);
         a.n = 0;
+        a.cols = 0;
     }
     return true;
 }

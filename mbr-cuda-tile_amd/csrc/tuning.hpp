@@ -65,6 +65,20 @@
 #ifndef MBRT_NT_CAT
 #define MBRT_NT_CAT 2    // concat of several sources in one launch
 #endif
+// Concat: sources of this average row and size, and so many bytes in all (beyond the 256 MB MALL with
+// the output), are copied one after another.  A launch apiece is little beside them, and a
+// thread's rows lie far apart: four f32 sources of 64 MB in rows of 16 MB 94 us one by one and 116 in
+// one launch, eight of 32 MB 103 and 109; but four of 32 MB 52 and 40, and two of 64 MB in rows of
+// 96 B 101 and 39.
+#ifndef MBRT_CAT_ROW
+#define MBRT_CAT_ROW (256ll << 10)  // bytes
+#endif
+#ifndef MBRT_CAT_SRC
+#define MBRT_CAT_SRC (24ll << 20)   // bytes
+#endif
+#ifndef MBRT_CAT_ALL
+#define MBRT_CAT_ALL (192ll << 20)  // bytes
+#endif
 #ifndef MBRT_NT_TR
 #define MBRT_NT_TR 0     // LDS tile transpose
 #endif

@@ -176,6 +176,34 @@ def test_cat_one_launch(orc, dev, outer, sizes, inner, dt, shift):
     assert_bitexact(to_host(out, dt), np.concatenate(parts, axis=1), "cat")
 
 
+# one odd view among aligned sources, rows just above and below one 16-byte vector, rows that are whole
+# vectors beside ones that are not, more sources than a launch holds, 8-byte elements off 16 bytes
+@pytest.mark.parametrize("outer,sizes,dt,shifts", [
+    (1, (4096, 4096), F32, (0, 1)), (1, (8192, 8193, 8191), BF16, (0, 3, 0)), (5, (4, 5, 7, 64), F32, (0, 0, 1, 2)),
+    (801, (8, 9, 15, 16, 17), BF16, (1, 0, 0, 5, 7)), (6, (7, 8), BF16, (0, 0)), (3, (3, 4), F32, (0, 0)),
+    (9, tuple(9 + i % 5 for i in range(130)), BF16, (0, 1)), (4, (2, 3, 11), I64, (1, 0, 1))])
+def test_cat_unaligned_sources(orc, dev, outer, sizes, dt, shifts):
+    say(f"cat unaligned outer={outer} sizes={sizes[:5]}x{len(sizes)} dt={dt} shifts={shifts}")
+    rng = np.random.default_rng(outer + 17 * len(sizes))
+    npdt = {F32: np.float32, BF16: np.uint16, I64: np.int64}[dt]
+    for out_shift in (0, 1):
+        parts, devs = [], []
+        for i, n in enumerate(sizes):
+            p = rng.integers(0, 2**15, size=(outer, n)).astype(npdt)
+            k = shifts[i % len(shifts)]
+            d = empty((p.size + k,), dt)[k:].view(outer, n)
+            d.copy_(to_dev(p, dt))
+            parts.append(p)
+            devs.append(d)
+        guard = 16
+        whole = torch.zeros(outer * sum(sizes) + out_shift + guard, dtype=devs[0].dtype, device="cuda")
+        out = whole[out_shift:-guard].view(outer, sum(sizes))
+        mbrt.cat(devs, 1, out)
+        torch.cuda.synchronize()
+        assert_bitexact(to_host(out, dt), np.concatenate(parts, axis=1), "cat")
+        assert not whole[:out_shift].any() and not whole[-guard:].any(), "written outside the output"
+
+
 # a source that lies in the output: what an earlier source has written there is what a later one
 # copies, as by one copy after another; and a source already in its place
 @pytest.mark.parametrize("n", [5, 1000, 300000])
