@@ -16,8 +16,8 @@
 //
 // STFT   one kernel: the workgroup's sample span ((kTF - 1) hop + 2048 samples, reflect
 //        padded at the signal ends) and the window are staged once into the frame slots
-//        with coalesced loads (hops up to 658; the span alone up to 950; larger hops read
-//        frame by frame), each wave takes its windowed frame from there, then FFT, real
+//        with coalesced loads (hops up to 658; larger hops read frame by frame), each wave
+//        takes its windowed frame from there, then FFT, real
 //        split, transposed store.  The split's 1/2 and the optional 1/sqrt(2048) scale the
 //        window.
 // iSTFT  two kernels: (1) per block of kTF frames of one signal: transposed spectrum load
@@ -365,7 +365,7 @@ struct StftArgs {
     uint32_t whole;    // groups that one workgroup takes whole
     int hop;
     int offset;        // 1024 when centred (reflect padding), else 0
-    int staged;        // the frame slots hold the workgroup's sample span (1), and the window too (2)
+    int staged;        // the frame slots hold the workgroup's sample span and the window
     float scale;       // 1/2 (of the real split), times 1/sqrt(2048) when normalized
 };
 
@@ -405,16 +405,15 @@ __device__ __forceinline__ float4 ld4_any(const float* p) { return __builtin_bit
 
 // Stages `span` (>= 2048) samples from sample s of signal xb into LDS, the even ones at xst and the
 // odd ones KH floats further (a frame's sample pairs are then two runs of consecutive words
-// whatever the frame's first sample), and the twiddles and (WIN) the scaled window beside
+// whatever the frame's first sample), and the twiddles and the scaled window beside
 // them.  Every load is in flight before the first LDS write where the span lies inside the
 // signal: KS vectors per thread, the vector index clamped to the last whole one.
-template <int KS, int KH, bool WIN>
+template <int KS, int KH>
 __device__ __forceinline__ void stage_span(const StftArgs& a, float* xst, float* wst, float2* tw, const float* xb, int s,
                                            int span) {
     const int tid = threadIdx.x;
     const float2 t = reinterpret_cast<const float2*>(kFftTable.v)[min(tid, kTwFwd - 1)];
-    float4 w = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if constexpr (WIN) w = ld4_any(a.w + 4 * tid);
+    const float4 w = ld4_any(a.w + 4 * tid);
     if (s >= 0 && s + span <= a.L) {
         const int last = (span >> 2) - 1, tail = min((span & ~3) + tid, span - 1);
         float4 xv[KS];
@@ -442,8 +441,7 @@ __device__ __forceinline__ void stage_span(const StftArgs& a, float* xst, float*
         }
     }
     if (tid < kTwFwd) tw[tid] = t;
-    if constexpr (WIN)
-        *reinterpret_cast<float4*>(wst + 4 * tid) = make_float4(w.x * a.scale, w.y * a.scale, w.z * a.scale, w.w * a.scale);
+    *reinterpret_cast<float4*>(wst + 4 * tid) = make_float4(w.x * a.scale, w.y * a.scale, w.z * a.scale, w.w * a.scale);
 }
 
 // Bound by vector arithmetic and LDS together, and by how evenly the CUs are loaded.  Per frame:
@@ -474,29 +472,22 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(MBRT_STFT_W
     const int s = (int)t0 * a.hop - a.offset;
     cf v[16];
     if (a.staged) {
-        // the frames of a workgroup overlap (hop < 2048): their span (and the window) are read
+        // the frames of a workgroup overlap (hop < 2048): their span and the window are read
         // from HBM once, coalesced, into the frame slots, and each wave takes its frame there
-        constexpr int KH2 = (kTF * kSlot - kN) / 2, KH1 = kTF * kSlot / 2;
-        float* xst = lds + (a.staged == 2 ? kN : 0);
+        constexpr int KH = (kTF * kSlot - kN) / 2;
+        float* xst = lds + kN;
         const int span = (nf - 1) * a.hop + kN;
-        if (a.staged == 2 && span <= 3 * 4 * kNT) stage_span<3, KH2, true>(a, xst, lds, tw, xb, s, span);
-        else if (a.staged == 2) stage_span<4, KH2, true>(a, xst, lds, tw, xb, s, span);
-        else stage_span<5, KH1, false>(a, xst, lds, tw, xb, s, span);
+        if (span <= 3 * 4 * kNT) stage_span<3, KH>(a, xst, lds, tw, xb, s, span);
+        else stage_span<4, KH>(a, xst, lds, tw, xb, s, span);
         __syncthreads();
         if (live) {
             // samples h + 2 m and h + 2 m + 1 of the span, h the frame's first
-            const int h = wave * a.hop, kh = a.staged == 2 ? KH2 : KH1;
-            const float* x0 = xst + (h & 1) * kh + (h >> 1) + lane;
-            const float* x1 = xst + (1 - (h & 1)) * kh + ((h + 1) >> 1) + lane;
+            const int h = wave * a.hop;
+            const float* x0 = xst + (h & 1) * KH + (h >> 1) + lane;
+            const float* x1 = xst + (1 - (h & 1)) * KH + ((h + 1) >> 1) + lane;
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
-                float2 w;
-                if (a.staged == 2) {
-                    w = reinterpret_cast<const float2*>(lds)[lane + 64 * q];
-                } else {
-                    w = ld2_any(a.w + 2 * (lane + 64 * q));
-                    w = make_float2(w.x * a.scale, w.y * a.scale);
-                }
+                const float2 w = reinterpret_cast<const float2*>(lds)[lane + 64 * q];
                 v[q] = cf{x0[64 * q] * w.x, x1[64 * q] * w.y};
             }
         }
@@ -934,10 +925,11 @@ int mbrt_stft(const float* signal, const float* window, float* out, int64_t batc
     a.hop = (int)hop;
     a.offset = center ? kN / 2 : 0;
     a.scale = normalized ? 0.5f / std::sqrt((float)kN) : 0.5f;
-    // what the kTF frame slots hold: the window and the span (hops up to 658), the span alone (up to
-    // 950), or neither: each wave then reads its frame from memory
-    const int64_t span = (kTF - 1) * hop + kN;
-    a.staged = kN + span <= kTF * kSlot ? 2 : span <= kTF * kSlot ? 1 : 0;
+    // the kTF frame slots hold the window and the span (hops up to 658), or each wave reads its
+    // frame from memory.  (Staging the span alone, which fits up to 950, and reading the window from
+    // memory ran [8, 352800] with a hop of 700 in 18.4 us instead of 15.2, [2, 352800] in 14.2
+    // instead of 10.5; whole complex slots, staged up to 1910, 15.7 and 10.9.)
+    a.staged = kN + (kTF - 1) * hop + kN <= kTF * kSlot ? 1 : 0;
     const int64_t groups = batch * ntb;
     MBRT_REQUIRE(groups < kMaxGridX, MBRT_E_SHAPE, "%s: too many frames", op);
     // A CU that gets one group more than the others sets the time, so the groups left over after
