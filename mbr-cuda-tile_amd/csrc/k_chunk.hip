@@ -11,10 +11,9 @@
 //
 // Memory-bound: per call C*n reads of src, C*n read-modify-writes of dest, n of the window
 // and n read-modify-writes of the weight sum.  A thread owns four sample positions
-// (of one channel, or of all channels for the normalize).  16-byte accesses at any sample
-// alignment: a song of odd length puts its second channel, and a chunk at an odd offset all of
-// its rows, off 16-byte addresses.  Per-sample kernels for those took 5.68 us per chunk of
-// [2, 352800] and 13.1 us to normalize [2, 2997817]; these take 4.9 and 12.1.
+// (of one channel, or of all channels for the normalize).  16-byte accesses also off 16-byte
+// addresses, where a song of odd length puts its second channel and a chunk at an odd offset all
+// of its rows, when there is much to move (MBRT_CHUNK_ANY).
 #include "abi_common.hpp"
 
 namespace mbrt {
@@ -44,6 +43,7 @@ struct AccArgs {
     int64_t dest_len;
     int64_t offset;
     int64_t channels;
+    uint32_t vblocks;     // blocks over whole vectors; one more takes the n % 4 samples left
 };
 
 // d + s w with the product rounded before the add (no contraction into an FMA).
@@ -52,40 +52,52 @@ __device__ __forceinline__ float acc1(float d, float s, float w) {
     return d + s * w;
 }
 
+__device__ __forceinline__ void accumulate1(const AccArgs& a, int64_t c, int64_t k, bool wsum) {
+    const float w = a.win[k];
+    float* d = a.dest + c * a.dest_len + a.offset + k;
+    *d = acc1(*d, a.src[c * a.n + k], w);
+    if (wsum) a.wsum[a.offset + k] = a.wsum[a.offset + k] + w;
+}
+
+// One sample per lane, a channel per grid row: unaligned chunks of few samples, where a
+// quarter of the waves with wider accesses take longer.
+__global__ __launch_bounds__(kThreads) void accumulate_scalar_kernel(AccArgs a) {
+    for (int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x; k < a.n; k += (int64_t)gridDim.x * kThreads)
+        accumulate1(a, blockIdx.y, k, blockIdx.y == 0);
+}
+
 // One wave per channel: a block of CPB waves takes channels [CPB y, CPB y + CPB) over the
 // same 64 consecutive 4-sample positions of the chunk, so the window's repeated reads are
-// made by waves of one CU, close together in time.  Positions are vectors of the chunk
-// (the last one may hold fewer than 4 samples): dest, weight sum and window addresses are
+// made by waves of one CU, close together in time.  Dest, weight sum and window addresses are
 // only sample-aligned where a song's length or a chunk's offset is odd, and 16-byte accesses
-// take that (ld_any).
+// take that (ld_any).  The samples after the last whole vector go to a block of their own: in
+// the vectors' loop one lane's three read-modify-writes held its wave for two more round trips.
 template <int CPB>
 __global__ __launch_bounds__(64 * CPB) void accumulate_cw_kernel(AccArgs a) {
     const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
     const int64_t c = (int64_t)blockIdx.y * CPB + w;
     const bool wsum = blockIdx.y == 0 && w == 0;
     if (c >= a.channels) return;
-    for (int64_t k = 4 * ((int64_t)blockIdx.x * 64 + lane); k < a.n; k += 4 * (int64_t)gridDim.x * 64) {
-        const float* sp = a.src + c * a.n + k;
+    if (blockIdx.x >= a.vblocks) {
+        const int64_t k = (a.n & ~int64_t(3)) + lane;
+        if (k < a.n) accumulate1(a, c, k, wsum);
+        return;
+    }
+    for (int64_t k = 4 * ((int64_t)blockIdx.x * 64 + lane); k + 4 <= a.n; k += 4 * (int64_t)a.vblocks * 64) {
         float* dp = a.dest + c * a.dest_len + a.offset + k;
-        float* wp = a.wsum + a.offset + k;
-        if (k + 4 <= a.n) {
-            const F4 wv = ld4<0>(a.win + k);
-            const F4 s = ld4<MBRT_NT_CHUNK & 1>(sp);
-            F4 d = ld4<MBRT_NT_CHUNK & 1>(dp);
+        const F4 wv = ld4<0>(a.win + k);
+        const F4 s = ld4<MBRT_NT_CHUNK & 1>(a.src + c * a.n + k);
+        F4 d = ld4<MBRT_NT_CHUNK & 1>(dp);
+        __builtin_amdgcn_sched_barrier(0);  // all three loads out before the first is waited for
 #pragma unroll
-            for (int e = 0; e < 4; ++e) d.v[e] = acc1(d.v[e], s.v[e], wv.v[e]);
-            st4<MBRT_NT_CHUNK & 2>(dp, d);
-            if (wsum) {
-                F4 ws = ld4<0>(wp);
+        for (int e = 0; e < 4; ++e) d.v[e] = acc1(d.v[e], s.v[e], wv.v[e]);
+        st4<MBRT_NT_CHUNK & 2>(dp, d);
+        if (wsum) {
+            float* wp = a.wsum + a.offset + k;
+            F4 ws = ld4<0>(wp);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) ws.v[e] = ws.v[e] + wv.v[e];
-                st4<0>(wp, ws);
-            }
-        } else {
-            for (int e = 0; e < (int)(a.n - k); ++e) {
-                dp[e] = acc1(dp[e], sp[e], a.win[k + e]);
-                if (wsum) wp[e] = wp[e] + a.win[k + e];
-            }
+            for (int e = 0; e < 4; ++e) ws.v[e] = ws.v[e] + wv.v[e];
+            st4<0>(wp, ws);
         }
     }
 }
@@ -140,12 +152,21 @@ int mbrt_chunk_accumulate(float* dest, float* weight_sum, const float* src, cons
                  (long long)(offset + chunk_len), (long long)dest_len);
     if (channels == 0 || chunk_len == 0) return MBRT_OK;
     MBRT_REQUIRE(dest && weight_sum && src && window, MBRT_E_INVALID_ARG, "%s: NULL pointer", op);
-    AccArgs a{dest, weight_sum, src, window, chunk_len, dest_len, offset, channels};
+    AccArgs a{dest, weight_sum, src, window, chunk_len, dest_len, offset, channels, 0};
     hipStream_t st = as_stream(stream);
     MBRT_REQUIRE(channels <= 65535, MBRT_E_SHAPE, "%s: too many channels", op);
+    // 16-byte accesses where all of them are aligned, and at any alignment where there is much to move
+    const bool vec = chunk_len % 4 == 0 && dest_len % 4 == 0 && offset % 4 == 0 && aligned(dest, 16) &&
+                     aligned(weight_sum, 16) && aligned(src, 16) && aligned(window, 16);
+    if (!vec && (chunk_len < 4 || channels * chunk_len < MBRT_CHUNK_ANY)) {
+        hipLaunchKernelGGL(accumulate_scalar_kernel, dim3((unsigned)grid_for(chunk_len), (unsigned)channels),
+                           dim3(kThreads), 0, st, a);
+        return check_launch(op);
+    }
     auto launch = [&](auto cpb) {
         constexpr int CPB = decltype(cpb)::value;
-        const unsigned gx = (unsigned)std::min<int64_t>(ceil_div(chunk_len, 256), int64_t(1) << 16);
+        a.vblocks = (uint32_t)std::min<int64_t>(ceil_div(chunk_len / 4, 64), int64_t(1) << 16);
+        const unsigned gx = a.vblocks + (chunk_len % 4 != 0 ? 1 : 0);
         hipLaunchKernelGGL(accumulate_cw_kernel<CPB>, dim3(gx, (unsigned)ceil_div(channels, CPB)), dim3(64 * CPB), 0, st,
                            a);
     };

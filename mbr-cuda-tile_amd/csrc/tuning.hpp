@@ -191,6 +191,13 @@
 #ifndef MBRT_CHUNK_CPB
 #define MBRT_CHUNK_CPB 4  // chunk accumulate: channels (one wave each) per block over shared positions (fewer when there are fewer channels)
 #endif
+// Chunk accumulate: samples over all channels from which unaligned chunks go in 16-byte accesses.  us per
+// call, one sample per lane against four, buffers warm: [2, 999] 2.53 and 3.10, [2, 44100] 2.90 and
+// 3.27, [2, 200002] 3.38 and 3.69, [8, 44100] 3.20 and 3.54; above: [2, 352800] 5.1 and 4.2, [4, 200002]
+// 5.3 and 4.3, [8, 352801] 10.5 and 9.0.
+#ifndef MBRT_CHUNK_ANY
+#define MBRT_CHUNK_ANY (1ll << 19)
+#endif
 #ifndef MBRT_EW_U
 #define MBRT_EW_U 4      // 16-byte groups per thread in the elementwise kernels
 #endif

@@ -44,6 +44,27 @@ def test_chunk_accumulate_and_normalize_bitexact(orc, dev, C, L, calls):
     assert_bitexact(to_host(dest, F32), dref, "normalize")
 
 
+# chunks off 16-byte addresses on both sides of the size where they go in 16-byte accesses, each
+# with 0 to 3 samples after the last whole vector, fewer channels than a block has waves and more
+@pytest.mark.parametrize("C,n", [(1, 3), (2, 1001), (1, 524287), (2, 262143), (2, 262145), (1, 524290), (3, 200003),
+                                 (5, 120004), (9, 60001)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_chunk_accumulate_unaligned_sizes(orc, dev, C, n, off):
+    say(f"chunk accumulate unaligned C={C} n={n} off={off}")
+    rng = np.random.default_rng(C * 31 + n)
+    L = n + 7
+    src = rng.standard_normal((C, n)).astype(np.float32)
+    win = rng.random(n).astype(np.float32)
+    dref = rng.standard_normal((C, L)).astype(np.float32)
+    wref = rng.random(L).astype(np.float32)
+    dest, ws = to_dev(dref, F32), to_dev(wref, F32)
+    mbrt.chunk_accumulate(dest, ws, to_dev(src, F32), to_dev(win, F32), off)
+    orc.chunk_accumulate(dref, wref, src, win, off)
+    torch.cuda.synchronize()
+    assert_bitexact(to_host(dest, F32), dref, "accumulate")
+    assert_bitexact(to_host(ws, F32), wref, "weight sum")
+
+
 def test_chunk_unaligned_views(orc, dev):
     """Offsets views into larger buffers: the scalar path handles any alignment."""
     say("chunk accumulate unaligned views")
