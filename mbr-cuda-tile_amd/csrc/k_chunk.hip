@@ -13,7 +13,7 @@
 // and n read-modify-writes of the weight sum.  A thread owns four sample positions
 // (of one channel, or of all channels for the normalize).  16-byte accesses also off 16-byte
 // addresses, where a song of odd length puts its second channel and a chunk at an odd offset all
-// of its rows, when there is much to move (MBRT_CHUNK_ANY).
+// of its rows, when there is much to move (MBRT_CHUNK_ANY, MBRT_NORM_ANY).
 #include "abi_common.hpp"
 
 namespace mbrt {
@@ -107,29 +107,41 @@ struct NormArgs {
     const float* __restrict__ wsum;  // [len]
     int64_t len;
     int64_t channels;
+    uint32_t vblocks;     // blocks over whole vectors; one more takes the len % 4 samples left
 };
 
 __device__ __forceinline__ float norm1(float v, float w) { return w > 1.0e-8f ? v / w : v; }
 
-// A thread owns 4 sample positions (the last one may hold fewer) and walks the channels, whose
-// rows are only sample-aligned where the length is not a multiple of 4.
+// One sample position per thread, walked over the channels.
+__global__ __launch_bounds__(kThreads) void normalize_scalar_kernel(NormArgs a) {
+    for (int64_t k = (int64_t)blockIdx.x * kThreads + threadIdx.x; k < a.len; k += (int64_t)gridDim.x * kThreads) {
+        const float w = a.wsum[k];
+        for (int64_t c = 0; c < a.channels; ++c) a.data[c * a.len + k] = norm1(a.data[c * a.len + k], w);
+    }
+}
+
+// A thread owns 4 sample positions and walks the channels, whose rows are only sample-aligned
+// where the length is not a multiple of 4.  The samples after the last whole vector go to a block
+// of their own, one (channel, sample) per thread: walked by one lane they took half of [16, 999].
 __global__ __launch_bounds__(kThreads) void normalize_vec_kernel(NormArgs a) {
-    for (int64_t k = 4 * ((int64_t)blockIdx.x * kThreads + threadIdx.x); k < a.len;
-         k += 4 * (int64_t)gridDim.x * kThreads) {
-        if (k + 4 <= a.len) {
-            const F4 w = ld4<0>(a.wsum + k);
+    if (blockIdx.x >= a.vblocks) {
+        const int64_t k0 = a.len & ~int64_t(3), tail = a.len - k0;
+        for (int64_t i = threadIdx.x; i < tail * a.channels; i += kThreads) {
+            const int64_t c = i / tail, k = k0 + i % tail;
+            a.data[c * a.len + k] = norm1(a.data[c * a.len + k], a.wsum[k]);
+        }
+        return;
+    }
+    for (int64_t k = 4 * ((int64_t)blockIdx.x * kThreads + threadIdx.x); k + 4 <= a.len;
+         k += 4 * (int64_t)a.vblocks * kThreads) {
+        const F4 w = ld4<0>(a.wsum + k);
 #pragma unroll 4
-            for (int64_t c = 0; c < a.channels; ++c) {
-                float* p = a.data + c * a.len + k;
-                F4 v = ld4<MBRT_NT_CHUNK & 1>(p);
+        for (int64_t c = 0; c < a.channels; ++c) {
+            float* p = a.data + c * a.len + k;
+            F4 v = ld4<MBRT_NT_CHUNK & 1>(p);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v.v[e] = norm1(v.v[e], w.v[e]);
-                st4<MBRT_NT_CHUNK & 2>(p, v);
-            }
-        } else {
-            for (int e = 0; e < (int)(a.len - k); ++e)
-                for (int64_t c = 0; c < a.channels; ++c)
-                    a.data[c * a.len + k + e] = norm1(a.data[c * a.len + k + e], a.wsum[k + e]);
+            for (int e = 0; e < 4; ++e) v.v[e] = norm1(v.v[e], w.v[e]);
+            st4<MBRT_NT_CHUNK & 2>(p, v);
         }
     }
 }
@@ -183,8 +195,15 @@ int mbrt_chunk_normalize(float* data, const float* weight_sum, int64_t channels,
     MBRT_REQUIRE(channels >= 0 && length >= 0, MBRT_E_SHAPE, "%s: negative extent", op);
     if (channels == 0 || length == 0) return MBRT_OK;
     MBRT_REQUIRE(data && weight_sum, MBRT_E_INVALID_ARG, "%s: NULL pointer", op);
-    NormArgs a{data, weight_sum, length, channels};
-    hipLaunchKernelGGL(normalize_vec_kernel, dim3((unsigned)grid_for(ceil_div(length, 4))), dim3(kThreads), 0,
+    NormArgs a{data, weight_sum, length, channels, (uint32_t)grid_for(length / 4)};
+    // as the accumulate: 16-byte accesses where aligned, and at any alignment where there is much to move
+    const bool vec = length % 4 == 0 && aligned(data, 16) && aligned(weight_sum, 16);
+    if (!vec && (length < MBRT_NORM_ANY || channels * length < 3 * MBRT_NORM_ANY)) {
+        hipLaunchKernelGGL(normalize_scalar_kernel, dim3((unsigned)grid_for(length)), dim3(kThreads), 0,
+                           as_stream(stream), a);
+        return check_launch(op);
+    }
+    hipLaunchKernelGGL(normalize_vec_kernel, dim3(a.vblocks + (length % 4 != 0 ? 1 : 0)), dim3(kThreads), 0,
                        as_stream(stream), a);
     return check_launch(op);
 }

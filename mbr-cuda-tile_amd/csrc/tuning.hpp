@@ -198,6 +198,15 @@
 #ifndef MBRT_CHUNK_ANY
 #define MBRT_CHUNK_ANY (1ll << 19)
 #endif
+// Chunk normalize: unaligned songs of this length, and of three times as many samples over all channels,
+// go in 16-byte accesses.  us per call, one position per thread against four: [2, 352801] 3.5 and 4.0,
+// [16, 352801] 11.2 and 15.4, [1, 1000003] 3.7 and 4.0; above: [2, 1000003] 6.1 and 5.5, [2, 2997817]
+// 13.0 and 11.8, or 18.8 and 11.9 with buffers out of cache, [8, 1000003] 19.0 and 13.9 out of cache.
+// The wide form's non-temporal accesses make no use of a warm cache: [8, 2997817] 35.1 and 38.1 warm, 51.1
+// and 39.2 out of cache.
+#ifndef MBRT_NORM_ANY
+#define MBRT_NORM_ANY (1ll << 19)
+#endif
 #ifndef MBRT_EW_U
 #define MBRT_EW_U 4      // 16-byte groups per thread in the elementwise kernels
 #endif

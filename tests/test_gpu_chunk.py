@@ -65,6 +65,21 @@ def test_chunk_accumulate_unaligned_sizes(orc, dev, C, n, off):
     assert_bitexact(to_host(ws, F32), wref, "weight sum")
 
 
+# normalize off 16-byte addresses on both sides of the sizes where it goes in 16-byte accesses
+@pytest.mark.parametrize("C,n", [(1, 1), (2, 3), (16, 999), (7, 5), (1, 524289), (3, 524287), (3, 524289), (4, 524290),
+                                 (2, 800003), (1, 1572865)])
+def test_chunk_normalize_unaligned_sizes(orc, dev, C, n):
+    say(f"chunk normalize unaligned C={C} n={n}")
+    rng = np.random.default_rng(C * 37 + n)
+    ref = rng.standard_normal((C, n)).astype(np.float32)
+    w = rng.random(n).astype(np.float32) - np.float32(0.25)  # some sums at or below the limit
+    data = to_dev(ref, F32)
+    mbrt.chunk_normalize(data, to_dev(w, F32))
+    torch.cuda.synchronize()
+    orc.chunk_normalize(ref, w)
+    assert_bitexact(to_host(data, F32), ref, "normalize")
+
+
 def test_chunk_unaligned_views(orc, dev):
     """Offsets views into larger buffers: the scalar path handles any alignment."""
     say("chunk accumulate unaligned views")
