@@ -191,6 +191,12 @@
 #ifndef MBRT_CHUNK_CPB
 #define MBRT_CHUNK_CPB 4  // chunk accumulate: channels (one wave each) per block over shared positions (fewer when there are fewer channels)
 #endif
+// Pads of 2-byte elements: elements written from which the kernel for whole rows takes them.  Eight of
+// them per thread leave few waves below: [64, 100 -> 200] 2.83 us an element per thread, 3.29 by rows;
+// [1000, 100 -> 200] 3.15 and 3.27, [2, 100000 -> 100200] 3.15 and 3.0.
+#ifndef MBRT_PAD2_MIN
+#define MBRT_PAD2_MIN (1ll << 16)
+#endif
 // Chunk accumulate: samples over all channels from which unaligned chunks go in 16-byte accesses.  us per
 // call, one sample per lane against four, buffers warm: [2, 999] 2.53 and 3.10, [2, 44100] 2.90 and
 // 3.27, [2, 200002] 3.38 and 3.69, [8, 44100] 3.20 and 3.54; above: [2, 352800] 5.1 and 4.2, [4, 200002]

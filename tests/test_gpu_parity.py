@@ -147,6 +147,15 @@ def test_pad_rows(orc, dev, dt, rows, n, before, m):
         assert_bitexact(to_host(out, dt), np.ascontiguousarray(ref.astype(x.dtype)), f"pad reflect={reflect}")
 
 
+# the same for 2-byte elements where there are enough of them to go by whole rows
+@pytest.mark.parametrize("rows,n,before,m", [(40, 1001, 500, 2001), (1700, 17, 3, 40), (5100, 5, 4, 13), (7300, 1, 2, 9),
+                                             (660, 100, 0, 100), (520, 64, 63, 190), (4200, 30, -7, 16), (550, 33, 40, 120),
+                                             (8200, 2, 1, 8), (1, 65000, 400, 70001)])
+def test_pad_rows_two_bytes(orc, dev, rows, n, before, m):
+    assert rows * m >= 1 << 16
+    test_pad_rows(orc, dev, dt=BF16, rows=rows, n=n, before=before, m=m)
+
+
 # (rows before the concat dim, source extents, elements after it, dtype, first-element offset of
 # the sources and the output): one column block, several, a row of columns just past one, more
 # sources than one launch holds, empty sources, every vector width, one row and many
