@@ -59,9 +59,9 @@ struct BiasActArgs {
 };
 
 // VE is 16 bytes of x and out (8 elements of two 2-byte operands, 4 when either is f32).  An f32
-// bias beside 2-byte operands is read as two vectors, being re-read from cache; going by its
-// width instead (4 elements, 8-byte accesses to x and out) ran [48060, 1536] bf16 GELU in
-// 64.0 us against 53.2, and is left for columns that are a multiple of 4 only.
+// bias beside 2-byte operands is read as two vectors, being re-read from cache, in large calls
+// (MBRT_BIAS_WIDE); in small ones, and where the columns are a multiple of 4 only, VE goes by its width
+// (4 elements, 8-byte accesses to x and out, twice the waves).
 template <int XDT, int ODT, int BDT, int ACT, int VE = (XDT == F32 || ODT == F32) ? 4 : 8>
 __global__ __launch_bounds__(kThreads) void bias_act_vec_kernel(BiasActArgs a) {
     constexpr bool LOWP = ODT != F32;
@@ -311,7 +311,8 @@ int mbrt_bias_act(const void* x, int x_dtype, const void* bias, int bias_dtype, 
                  "%s: in-place needs equal element sizes", op);
     hipStream_t st = as_stream(stream);
     const bool lowp = x_dtype != F32 && out_dtype != F32;
-    const bool narrow = lowp && bias != nullptr && bias_dtype == F32 && cols % 8 != 0;
+    const int64_t wide = act == MBRT_ACT_GELU_REF || act == MBRT_ACT_GELU_STD ? MBRT_BIAS_WIDE_GELU : MBRT_BIAS_WIDE;
+    const bool narrow = lowp && bias != nullptr && bias_dtype == F32 && (cols % 8 != 0 || a.n < wide);
     const int ve = lowp && !narrow ? 8 : 4;
     const bool vec = aligned(x, 16) && aligned(out, 16) &&
                      (bias == nullptr || (aligned(bias, 16) && cols % ve == 0 && a.n < (1ll << 32)));

@@ -532,6 +532,24 @@ def test_bias_act_f32_bias_widths(orc, dev, rows, cols, dt):
         assert_close(to_host(y, dt), orc.bias_act(x, dt, b, F32, dt, act), dt, f"act {act}")
 
 
+# the same at sizes whose f32 bias goes with 16-byte accesses (and, just below, with 8-byte ones): each
+# call over the whole against calls over its two halves, which are below the limit
+@pytest.mark.parametrize("rows,cols,act", [(8193, 1024, 3), (5462, 1544, 4), (8191, 1024, 4), (32769, 1024, 1),
+                                           (21848, 1536, 2)])
+def test_bias_act_f32_bias_large(dev, rows, cols, act):
+    say(f"bias_act f32 bias whole and halves rows={rows} cols={cols} act={act}")
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn((rows, cols), generator=g, device="cuda").to(torch.bfloat16)
+    b = torch.randn(cols, generator=g, device="cuda")
+    y, z = torch.empty_like(x), torch.empty_like(x)
+    mbrt.bias_act(x, b, y, act)
+    h = rows // 2
+    mbrt.bias_act(x[:h], b, z[:h], act)
+    mbrt.bias_act(x[h:], b, z[h:], act)
+    torch.cuda.synchronize()
+    assert torch.equal(y, z)
+
+
 def test_glu_bl2b_full(orc, dev):
     say("BL-2b GLU bf16 [48060,3072]")
     x = inp(orc, (48060, 3072), SEED[2], 2, BF16, std=1.5)
