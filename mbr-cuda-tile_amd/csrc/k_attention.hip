@@ -682,20 +682,22 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(HEA
 // ones also pad less.  Measured (us, 32 -> 16 queries per wave, P pair):
 //   c2 = 1                [8, 801] 18.7 -> 12.8, [60, 401] 12.6 -> 10.8, [120, 200] 9.0 -> 8.0
 //   c1 <= 2 c2 - c2 / 4   [48, 801] (2, 3) 27.9 -> 23.0, [480, 150] (4, 6) 17.1 -> 14.8,
-//                         [480, 300] (6, 10) 32.1 -> 29.8, [480, 401] (8, 14) 51.9 -> 48.8
+//                         [480, 280] (6, 10) 31.5 -> 29.7, [480, 300] 32.7 -> 31.8
 //   above                 [60, 801] (2, 4) 25.9 -> 27.1, [120, 1601] (7, 13) 140 -> 149
+//   c2 = 8 and more       [480, 401] (8, 14) 51.8 -> 55.4, [480, 430] 52.6 -> 54.9, [512, 400] 49.2 -> 50.7
 // The single-P modes, with less arithmetic per fragment, need half the margin more: [240, 401]
 // (4, 7) 31.0 -> 29.3 as a pair but 22.1 -> 23.1 fast; [48, 801] 21.2 -> 17.8 fast.  A tie (c1 =
-// 2 c2 <= 4) goes to 16 where there are few key tiles and the 64-query workgroups are mostly
-// full: [480, 101] fast 8.4 -> 7.9, [480, 128] 9.4 -> 8.5, but [480, 70] pair 7.7 -> 8.1.
+// 2 c2 <= 4) goes to 16 where there are one or two key tiles and the 64-query workgroups are mostly
+// full: [480, 101] fast 8.4 -> 7.9, [480, 128] 9.4 -> 8.5, but [480, 70] pair 7.7 -> 8.1 and, over four
+// key tiles, [256, 256] pair 13.2 -> 13.5.
 bool narrow_queries(int64_t BH, int64_t n_q, int64_t n_k, bool pair) {
     const int64_t cus = cu_count();
     const int64_t t1 = ceil_div(n_q, kQBlock), t2 = ceil_div(n_q, 2 * kQBlock);
     const int64_t c1 = ceil_div(BH * t1, cus), c2 = ceil_div(BH * t2, cus);
     if (c2 == 1) return true;
-    if (c2 > 8) return false;
+    if (c2 >= 8) return false;
     if (c1 + ceil_div(c2, pair ? 4 : 2) <= 2 * c2) return true;
-    return c2 == 2 && n_k <= 4 * kKeys && 4 * n_q >= 3 * kQBlock * t1;
+    return c2 == 2 && n_k <= 2 * kKeys && 4 * n_q >= 3 * kQBlock * t1;
 }
 
 }  // namespace
