@@ -33,6 +33,7 @@ __device__ __forceinline__ void st4(float* p, const F4& x) {
 }
 
 constexpr int kThreads = 256;
+static_assert(MBRT_CHUNK_CPB >= 1 && MBRT_CHUNK_CPB <= 16, "one wave per channel, 1 to 16 of them in a block");
 
 struct AccArgs {
     float* __restrict__ dest;       // [C, dest_len]

@@ -189,7 +189,7 @@
 #define MBRT_GATE_BPC 16  // sigmoid gate x head merge: blocks per CU of a grid that walks the chunks (0: one chunk per block)
 #endif
 #ifndef MBRT_CHUNK_CPB
-#define MBRT_CHUNK_CPB 4  // chunk accumulate: channels (one wave each) per block over shared positions (fewer when there are fewer channels)
+#define MBRT_CHUNK_CPB 4  // chunk accumulate: channels (one wave each) per block over shared positions, 1 to 16 (fewer when there are fewer channels)
 #endif
 // Bias + activation with an f32 bias beside 2-byte operands: elements from which a thread takes 16 bytes
 // of those.  us, 8 bytes against 16, buffers warm up to 256 MB of them: GELU [400, 384] 2.66 and 2.95,

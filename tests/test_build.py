@@ -3,6 +3,7 @@ The compiler is stood in for by a function that records its output files."""
 from __future__ import annotations
 
 import importlib.util
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -54,3 +55,13 @@ def test_build_error_in_the_extension_comes_after_the_libraries(pkg_build, tmp_p
     with pytest.raises(RuntimeError, match="command failed"):
         pkg_build.build(out_dir=tmp_path)
     assert (tmp_path / "libmbrt.so").exists() and (tmp_path / "libmbrt_tensor.so").exists()
+
+
+@pytest.mark.parametrize("cpb,ok", [(0, False), (17, False), (1, True)])
+def test_chunk_channels_per_block_out_of_range_do_not_build(pkg_build, cpb, ok):
+    """A block of no waves, or of more than 1024 threads, is refused when it is compiled."""
+    cmd = [pkg_build.HIPCC, *pkg_build.COMMON, f"-DMBRT_CHUNK_CPB={cpb}", "-x", "hip", "--cuda-host-only",
+           "-fsyntax-only", str(PKG / "csrc" / "k_chunk.hip")]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert (r.returncode == 0) == ok, r.stderr
+    assert ok or "one wave per channel" in r.stderr
