@@ -97,7 +97,9 @@ __global__ __launch_bounds__(kThreads) void softmax_rows_kernel(SmArgs a) {
 // stores the span.  In-place calls are safe: the whole span is in LDS before its first
 // store.
 // HOT: the input is small enough to be cached (see MBRT_HOT_BYTES) and loaded by ordinary
-// loads.  (An instance of its own: the choice at run time cost the time softmax 0.2 %.)
+// loads.  (An instance of its own: the choice at run time cost the time softmax 0.2 %.  Only for
+// equal types outside the full-bf16 mode: the others would double the instances for calls that
+// the path does not make.)
 template <int IDT, int ODT, int G, int NM, int RPG, bool FB, bool HOT = false>
 __global__ __launch_bounds__(kThreads) void softmax_staged_kernel(SmArgs a) {
     constexpr int RB = RPG * kThreads / G;

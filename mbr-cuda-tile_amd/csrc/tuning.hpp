@@ -9,25 +9,32 @@
 //             policies 0..3 per kernel, the best kept; differences under ~3 % are noise.
 #pragma once
 
-// Inputs of up to MBRT_HOT_BYTES bytes are read with ordinary loads whatever the policy says:
-// an input that small has usually just been written and still sits in the 256 MB MALL (or an
-// L2), which non-temporal loads make no use of.  Each kernel over two cycled buffer sets: split +
-// rotary of 18.6 MB 8.35 -> 6.21 us, gate merge of 12.3 MB 6.19 -> 4.28, permute of 18.5 MB
-// 8.24 -> 7.04, f32 softmax [4000, 801] 5.11 -> 4.58, bf16 rows of 60 columns 2.87 -> 2.64.  Larger
-// inputs gain as much while they are warm (split of 37 MB 14.5 -> 12.1), but in a chain of calls they
-// are cold by then and lose: the token step of 401 frames 61.6 -> 62.9 us with 40 MB as the limit.
-// RMSNorm and GLU, whose second operands come from further back, take MBRT_HOT_BYTES_ACT:
-// with 20 MB the token step of 201 frames ran 33.9 -> 34.9 us over three buffer sets.  The gate merge
-// takes MBRT_HOT_BYTES_GATE: in the frequency attention's chain of calls, 12.3 MB into it ([200, 60]
-// rows) ran 31.8 us with ordinary loads and 31.2 without, 18.4 MB 44.8 and 43.2.
+// The softmax and the qkv split read inputs of up to MBRT_HOT_BYTES bytes with ordinary loads, whatever
+// their policy says, and the gate merge attention values of up to MBRT_HOT_BYTES_GATE: an input that
+// small has usually just been written and still sits in the 256 MB MALL (or an L2), which non-temporal
+// loads make no use of.  us per call with non-temporal and with ordinary loads, two buffer sets in turn
+// (warm), and twelve (cold up to the sizes given last in each row):
+//                                            warm           cold
+//   split + rotary, 18.6 MB of qkv        8.65   7.04     8.96   7.29
+//                   37 MB                14.7   12.6     15.3   15.9
+//   gate merge, 6.2 MB of attention       4.03   3.52     4.03   4.18
+//               24.6 MB                   9.64   8.95    10.8   11.2
+//   softmax f32 [4000, 801], 12.8 MB      5.80   4.99     6.09   5.87
+//               [12000, 801], 38 MB      17.2   13.0     17.3   17.7
+// The lines lie where the attention layer's three calls stop gaining when its buffers are cold (two
+// sets in turn, and six):
+//   [60, 110], qkv 20.3 MB, gate 6.8     22.4   20.2     22.6   22.7
+//   [60, 120], qkv 22.1 MB (split only)  23.6   21.2     23.4   24.3
+//   [60, 150], qkv 27.6 MB, gate 9.2     30.9   27.9     30.2   32.4
+//   [200, 60], qkv 36.9 MB, gate 12.3    31.1   29.3     30.9   31.8
+// Row copies, RMSNorm and GLU keep their policy at every size: by ordinary loads of the small ones the
+// token step took 13.4 -> 14.8 us at 45 frames (two sets) and 25.1 -> 27.4 at 130 (six), for
+// 25.2 -> 23.6 at 130 with two.
 #ifndef MBRT_HOT_BYTES
 #define MBRT_HOT_BYTES (20ll << 20)
 #endif
 #ifndef MBRT_HOT_BYTES_GATE
 #define MBRT_HOT_BYTES_GATE (8ll << 20)
-#endif
-#ifndef MBRT_HOT_BYTES_ACT
-#define MBRT_HOT_BYTES_ACT (12ll << 20)
 #endif
 #ifndef MBRT_NT_RMS
 #define MBRT_NT_RMS 3    // residual add + RMSNorm: x, residual, sum, normed
