@@ -394,10 +394,11 @@ def test_reductions(orc, dev):
 # ---- cache policy by input size ------------------------------------------------------------
 
 # Inputs just below and above the sizes where the streaming kernels change their load policy
-# (12 MB for RMSNorm and GLU, 20 MB for the others) give the same results: each call over the
-# large input against calls over its two halves
+# (20 MB for softmax and the qkv split, 8 MB of attention values for the gate merge; the others
+# have one policy) give the same results: each call over the large input against calls over
+# its two halves
 def test_load_policy_changes_no_result(dev):
-    say("load policy: whole inputs of 12..24 MB against their halves")
+    say("load policy: whole inputs of 9..40 MB against their halves")
     g = torch.Generator(device="cuda").manual_seed(11)
     rnd = lambda *s, dt=torch.bfloat16: torch.randn(s, generator=g, device="cuda").to(dt)  # noqa: E731
     gamma = torch.ones(384, device="cuda")
@@ -434,6 +435,7 @@ def test_load_policy_changes_no_result(dev):
     halves(rms, 4100, rnd(8300, 384), rnd(8300, 384))
     halves(glu, 1024, rnd(2052, 3072))
     halves(gate, 12, rnd(26, 8, 801, 64), rnd(26, 801, 8))
+    halves(gate, 6, rnd(12, 8, 801, 64), rnd(12, 801, 8))  # 9.8 MB against 4.9 and 4.9
     halves(softmax, 6552, rnd(13128, 801))
     halves(softmax, 3276, rnd(6564, 801, dt=torch.float32))
     halves(softmax, 90000, rnd(180000, 60))
