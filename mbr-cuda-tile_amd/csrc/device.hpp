@@ -352,8 +352,6 @@ __device__ __forceinline__ void gst(T* p, T v) {
     else *p = v;
 }
 
-// 16 bytes at an address aligned to A bytes only (A = 4 or 2): one dwordx4 access, which
-// global memory takes at any alignment (unaligned access mode, the default of HSA code).
 // Issues a kernel's streaming loads, f(std::integral_constant<int, policy>), by policy NT when
 // `cold` (uniform), else with ordinary loads.  The empty asm statements keep the compiler from
 // merging the two branches' loads into one set, which drops the non-temporal bit.
@@ -370,6 +368,8 @@ __device__ __forceinline__ void load_by(int cold, F f) {
     }
 }
 
+// 16 bytes at an address aligned to A bytes only (A = 4 or 2): one dwordx4 access, which
+// global memory takes at any alignment (unaligned access mode, the default of HSA code).
 template <int A>
 struct AnyVec;
 template <> struct AnyVec<4> { typedef uint32_t T __attribute__((ext_vector_type(4), aligned(4))); };

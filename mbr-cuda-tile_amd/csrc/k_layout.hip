@@ -111,8 +111,9 @@ __global__ __launch_bounds__(kThreads) void row_copy_kernel(RowCopyArgs a) {
 // at the row's end, so that it rewrites a few of the previous vector's bytes with the same
 // values.  A is the alignment that all rows have.  Copying with words of that size instead
 // is bound by the number of accesses: the 18 slice copies of a one-minute song's chunks
-// ([2, 352800] f32 and the final crop of [2, 2645017]) took 4.79 us on average, now 3.37-3.40
-// (3.7 with ordinary stores, 3.8-4.0 non-temporal both ways); the crop alone 14.8 -> 11.
+// ([2, 352800] f32 and the final crop of [2, 2645017]) took 4.85 us on average, now 3.58: the
+// whole slices 4.37 -> 3.22, the crop 14.5 -> 9.8.  (All of them with ordinary stores 9 % more, with
+// non-temporal loads as well 14 %.)
 struct RowCopyUArgs {
     RowCopyArgs r;
     int64_t last;  // offset of a row's last vector: row bytes - 16
@@ -555,7 +556,7 @@ __global__ __launch_bounds__(kThreads) void pad_kernel(PadArgs a) {
 // as in row_copy_any_kernel) from one 16-byte load wherever its elements are all inside the
 // source or, reversed, all inside one reflected border; the few vectors across an edge go
 // element by element.  The general kernel divides in 64 bits per element and dim: the reflect
-// pad of a [1, 2, 2645017] f32 song took 34.2 us, here 12.3-13.
+// pad of a [1, 2, 2645017] f32 song took 32.3 us, here 9.8.
 struct PadRowArgs {
     const char* src;
     char* dst;

@@ -61,8 +61,8 @@ constexpr int kSub = MBRT_STFT_SUB;         // frames of an STFT workgroup that 
 #define MBRT_ISTFT_WPE 4
 #endif
 // MBRT_STFT_WPE, MBRT_ISTFT_WPE: waves per SIMD the register budgets allow for at least.  The STFT
-// needs 70 VGPRs (three workgroups, 24 waves, per CU by registers).  Held to 64 for four, it
-// spills 28 bytes a lane: 21.7 us against 21.4 on the chunk.
+// needs 64 VGPRs (four workgroups, 32 waves, per CU by registers and LDS), the iSTFT's block kernel 78 and
+// twice the LDS (two workgroups).
 //
 // Frame blocks are dealt to the XCDs in runs of this many consecutive blocks, so the blocks
 // that share the cache lines of a bin row ([B, 1025, T] holds kTF frames of a bin in
@@ -445,11 +445,13 @@ __device__ __forceinline__ void stage_span(const StftArgs& a, float* xst, float*
 }
 
 // Bound by vector arithmetic and LDS together, and by how evenly the CUs are loaded.  Per frame:
-// 826 vector instructions (8.6 us of SIMD time on the chunk, [8, 352800] -> 6,408 frames) and 685
-// LDS cycles (7.1 us), beside 64 MB of HBM (11 us).  The kernel that kept whole complex slots (two
-// workgroups per CU) and computed its twiddle indices took 1,111 and 720 cycles, of which 153 were bank
-// conflicts: 25.5 us.  Half slots, per-lane twiddle tables and layouts without conflicts: 21.4.
-// The same with layouts padded by p/16, whose 32-bit reads conflict: 28.4.
+// 837 vector instructions (8.7 us of SIMD time on the chunk, [8, 352800] -> 6,408 frames) and 729
+// LDS cycles (7.6 us), beside 64 MB of HBM (11 us).  65 of the LDS cycles are bank conflicts: the
+// exchanges, the window, the twiddles and the transposed accesses have none by their indices, so
+// they are likely the staging's, whose surplus threads all write the span's last vector again.
+// The kernel that kept whole complex slots (two workgroups per CU) and computed its twiddle indices
+// took 1,121 instructions and 726 cycles, of which 154 were conflicts.  25.7 us then, 19.7 now
+// (rocprofv3, one box).  The same with layouts padded by p/16, whose 32-bit reads conflict: 28.4.
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(MBRT_STFT_WPE))) void stft_kernel(StftArgs a) {
     __shared__ __attribute__((aligned(16))) float lds[kTF * kSlot + 2 * kTwFwd];
     float2* tw = reinterpret_cast<float2*>(lds + kTF * kSlot);
@@ -639,10 +641,10 @@ __device__ __forceinline__ cf c2r_bin(float2 xk, float2 xg, float c, float s) {
 }
 
 // Bound by its chain of phases: load, inverse split, FFT, window, overlap-add, with two
-// workgroups per CU by LDS.  Per frame 1,050 vector instructions (1,410 before) and 624 LDS cycles
-// (830 before), no bank conflicts.  Chunk [8, 1025, 801] f32: 29.6 -> 27.2 us; two signals of 620
-// frames, bf16, 156 workgroups: 12.4 -> 10.9.  Half slots as the STFT's, with the spectra and the
-// overlap-add in two rounds each (four workgroups per CU), ran 27.5 and 13.5.
+// workgroups per CU by LDS.  Per frame 1,042 vector instructions (1,422 before) and 653 LDS cycles
+// (837 before), no bank conflicts.  Chunk [8, 1025, 801] f32: 29.9 -> 28.0 us; two signals of 620
+// frames, bf16, 156 workgroups: 12.0 -> 11.6 to 12.0.  Half slots as the STFT's, with the spectra
+// and the overlap-add in two rounds each (four workgroups per CU), ran 0.3 and 2.6 us longer.
 template <int SDT>
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(MBRT_ISTFT_WPE))) void istft_block_kernel(IstftBlockArgs a) {
     typedef typename SpecElem<SDT>::T Elem;
