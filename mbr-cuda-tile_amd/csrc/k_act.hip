@@ -123,6 +123,7 @@ struct GluArgs {
     int64_t rows, half;
     int64_t groups;   // rows * half / VE
     FastDiv gpr;      // groups per row = half / VE
+    int cold;         // the input is too large to be cached
     int fb;           // bf16 intermediates (element kernel; the vector kernel takes FB)
 };
 
@@ -131,14 +132,17 @@ __global__ __launch_bounds__(kThreads) void glu_vec_kernel(GluArgs a) {
     constexpr int VE = (XDT == F32 || ODT == F32) ? 4 : 8;
     const int64_t base = (int64_t)blockIdx.x * (kThreads * kUGlu) + threadIdx.x;
     Vec<XDT, VE> xv[kUGlu], gv[kUGlu];
+    load_by<MBRT_NT_GLU>(a.cold, [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
 #pragma unroll
-    for (int u = 0; u < kUGlu; ++u) {
-        uint32_t row, c;
-        fdivmod((uint32_t)clamp_group(base + u * kThreads, a.groups), a.gpr, row, c);
-        const int64_t in0 = (int64_t)row * (2 * a.half) + (int64_t)c * VE;
-        xv[u].template load<MBRT_NT_GLU>(a.x, in0);
-        gv[u].template load<MBRT_NT_GLU>(a.x, in0 + a.half);
-    }
+        for (int u = 0; u < kUGlu; ++u) {
+            uint32_t row, c;
+            fdivmod((uint32_t)clamp_group(base + u * kThreads, a.groups), a.gpr, row, c);
+            const int64_t in0 = (int64_t)row * (2 * a.half) + (int64_t)c * VE;
+            xv[u].template load<NT>(a.x, in0);
+            gv[u].template load<NT>(a.x, in0 + a.half);
+        }
+    });
 #pragma unroll
     for (int u = 0; u < kUGlu; ++u) {
         const int64_t g = base + u * kThreads;
@@ -363,6 +367,7 @@ int mbrt_glu_last_dim(const void* x, int x_dtype, void* out, int out_dtype, int6
     if (vec) {
         a.groups = rows * half_dim / ve;
         a.gpr = make_fastdiv((uint32_t)(half_dim / ve));
+        a.cold = cold_input(2 * rows * half_dim * dt_size(x_dtype), MBRT_HOT_BYTES_ACT);
         with_dt(x_dtype, [&](auto xt) {
             with_dt(out_dtype, [&](auto ot) {
                 constexpr int X = decltype(xt)::value, O = decltype(ot)::value;

@@ -70,6 +70,7 @@ struct RowCopyArgs {
     FastDiv vpr;             // vectors per row
     int64_t dst_pitch;       // output row pitch in bytes
     int nd;                  // number of outer dims
+    int cold;                // the source is too large to be cached
     FastDiv outer[kMaxOuter];        // outer dim extents, innermost first
     int64_t outer_stride[kMaxOuter]; // source pitch in bytes, innermost first
 };
@@ -79,7 +80,7 @@ __global__ __launch_bounds__(kThreads) void row_copy_kernel(RowCopyArgs a) {
     typedef typename WordOf<W>::T Word;
     const uint32_t base = blockIdx.x * (kThreads * U) + threadIdx.x;
     Word v[U];
-    int64_t dst_off[U];
+    int64_t dst_off[U], src_off[U];
     // all loads first (index clamped into the copy), then predicated stores
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -97,8 +98,12 @@ __global__ __launch_bounds__(kThreads) void row_copy_kernel(RowCopyArgs a) {
                 row = q;
             }
         }
-        v[u] = gld<MBRT_NT_ROW>(reinterpret_cast<const Word*>(a.src + off));
+        src_off[u] = off;
     }
+    load_by<MBRT_NT_ROW>(a.cold, [&](auto nt) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = gld<decltype(nt)::value>(reinterpret_cast<const Word*>(a.src + src_off[u]));
+    });
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         if (base + u * kThreads < a.total_vec) gst<MBRT_NT_ROW>(reinterpret_cast<Word*>(a.dst + dst_off[u]), v[u]);
@@ -189,6 +194,7 @@ int launch_row_copy(const char* src, char* dst, const Dims& dm, int esize, int64
         a.vpr = make_fastdiv((uint32_t)vpr);
         a.dst_pitch = dst_pitch;
         a.nd = dm.nd - 1;
+        a.cold = cold_input(total * W);
         for (int d = 0; d < a.nd; ++d) {
             int src_d = dm.nd - 2 - d;
             a.outer[d] = make_fastdiv((uint32_t)dm.shape[src_d]);

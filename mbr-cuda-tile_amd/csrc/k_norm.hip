@@ -39,6 +39,7 @@ struct RmsArgs {
     float scale;
     float eps;
     int fb;      // bf16 intermediates (loop kernel; the fast kernel takes it as FB)
+    int cold;    // the input is too large to be cached: its loads go by the kernel's policy
 };
 
 // One block = 256 / G rows.  gamma * scale is staged once per block in LDS as f32.  The
@@ -57,12 +58,15 @@ __global__ __launch_bounds__(kThreads) void rms_fast_kernel(RmsArgs a) {
     const int64_t base = (valid ? row : a.rows - 1) * a.dim;
     const int lastc = a.nchunk - 1;
     Vec<XDT, VE> xv[NC], rv[NC];
+    load_by<MBRT_NT_RMS>(a.cold, [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
 #pragma unroll
-    for (int k = 0; k < NC; ++k) {
-        const int c = min(lane + G * k, lastc);
-        xv[k].template load<MBRT_NT_RMS>(a.x, base + c * VE);
-        if (RES) rv[k].template load<MBRT_NT_RMS>(a.res, base + c * VE);
-    }
+        for (int k = 0; k < NC; ++k) {
+            const int c = min(lane + G * k, lastc);
+            xv[k].template load<NT>(a.x, base + c * VE);
+            if (RES) rv[k].template load<NT>(a.res, base + c * VE);
+        }
+    });
     for (int d = threadIdx.x; d < a.dim; d += kThreads)
         gs[d] = FB ? bf16r(load1(a.gamma, a.gdt, d)) : load1(a.gamma, a.gdt, d) * a.scale;
     float v[NC][VE];
@@ -178,6 +182,8 @@ int launch_rms(RmsArgs a, hipStream_t st, const char* op) {
     a.fb = bf16_intermediates() && a.odt == BF16;
     const int ve = (a.xdt == F32 || a.odt == F32) ? 4 : 8;
     const bool res = a.res != nullptr;
+    // (2-byte inputs gain nothing in the token step from ordinary loads)
+    a.cold = a.xdt != F32 || cold_input(a.rows * a.dim * dt_size(a.xdt) * (res ? 2 : 1), MBRT_HOT_BYTES_ACT);
     const bool al = aligned(a.x, 16) && aligned(a.out, 16) && (!res || aligned(a.res, 16)) &&
                     (a.sum_out == nullptr || aligned(a.sum_out, 16));
     // the fused path stores the residual sum in the input dtype

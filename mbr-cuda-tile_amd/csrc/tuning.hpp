@@ -9,9 +9,10 @@
 //             policies 0..3 per kernel, the best kept; differences under ~3 % are noise.
 #pragma once
 
-// The softmax and the qkv split read inputs of up to MBRT_HOT_BYTES bytes with ordinary loads, whatever
-// their policy says, and the gate merge attention values of up to MBRT_HOT_BYTES_GATE: an input that
-// small has usually just been written and still sits in the 256 MB MALL (or an L2), which non-temporal
+// Small inputs are read with ordinary loads, whatever a kernel's policy says: up to MBRT_HOT_BYTES bytes
+// by the softmax, the qkv split and the row copy, up to MBRT_HOT_BYTES_GATE of attention values by the
+// gate merge, up to MBRT_HOT_BYTES_ACT by the GLU and, of f32, by RMSNorm.  An input that small has
+// usually just been written and still sits in the 256 MB MALL (or an L2), which non-temporal
 // loads make no use of.  us per call with non-temporal and with ordinary loads, two buffer sets in turn
 // (warm), and twelve (cold up to the sizes given last in each row):
 //                                            warm           cold
@@ -27,14 +28,24 @@
 //   [60, 120], qkv 22.1 MB (split only)  23.6   21.2     23.4   24.3
 //   [60, 150], qkv 27.6 MB, gate 9.2     30.9   27.9     30.2   32.4
 //   [200, 60], qkv 36.9 MB, gate 12.3    31.1   29.3     30.9   31.8
-// Row copies, RMSNorm and GLU keep their policy at every size: by ordinary loads of the small ones the
-// token step took 13.4 -> 14.8 us at 45 frames (two sets) and 25.1 -> 27.4 at 130 (six), for
-// 25.2 -> 23.6 at 130 with two.
+// In the token step of T frames (permute, RMSNorm, GELU, GLU; bf16, 384 features) each kernel's share
+// goes with what the chain's buffers hold in all.  Step by ordinary loads in one kernel over the step
+// without any, one / two / three / six sets in turn:
+//                  row copy                  GLU                       RMSNorm
+//   T =  50   .98  1.07  .99  .98      .98  1.07 1.00  .99      1.02 1.11 1.05 1.02
+//   T =  90  1.01   .98  .98  .99     1.03   .99  .99  .99      1.07  .99  .99 1.01
+//   T = 130   .97   .97  .97  .97      .97   .97  .97  .97      1.01 1.00 1.00 1.00
+//   T = 201   .96   .99  .98 1.06      .96   .99  .97 1.10       .97  .99  .98 1.10
+// RMSNorm of 2-byte inputs has the losses without the gain and keeps its policy; of f32, 192 features,
+// it gains (T = 100: 1.02 .95 .95 .95).  12 MB of GLU input are T = 136.
 #ifndef MBRT_HOT_BYTES
 #define MBRT_HOT_BYTES (20ll << 20)
 #endif
 #ifndef MBRT_HOT_BYTES_GATE
 #define MBRT_HOT_BYTES_GATE (8ll << 20)
+#endif
+#ifndef MBRT_HOT_BYTES_ACT
+#define MBRT_HOT_BYTES_ACT (12ll << 20)
 #endif
 #ifndef MBRT_NT_RMS
 #define MBRT_NT_RMS 3    // residual add + RMSNorm: x, residual, sum, normed
