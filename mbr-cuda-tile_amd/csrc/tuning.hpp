@@ -210,15 +210,16 @@
 #define MBRT_CHUNK_CPB 4  // chunk accumulate: channels (one wave each) per block over shared positions, 1 to 16 (fewer when there are fewer channels)
 #endif
 // Bias + activation with an f32 bias beside 2-byte operands: elements from which a thread takes 16 bytes
-// of those.  us, 8 bytes against 16, buffers warm up to 256 MB of them: GELU [400, 384] 2.66 and 2.95,
-// [3000, 1536] 5.8 and 6.2, [12000, 384] 5.7 and 6.2, [36000, 768] 22.0 and 22.7; [24000, 1536] 28.4 and
-// 28.2, [48060, 1536] 61 and 54 (rocprofv3, out of cache: 64 and 54), [96120, 768] 60 and 54.  Tanh
-// [3000, 1536] 7.0 and 7.7, [12000, 1536] 18.3 and 17.1; sigmoid 5.4 and 5.2, 13.6 and 12.3.
+// of those.  us, 8 bytes against 16: GELU [400, 384] 2.66 and 2.95, [3000, 1536] 5.8 and 6.2, [12000, 384]
+// 5.7 and 6.2, [9000, 1024] 8.8 and 9.1; from 17 to 37 million elements within 4 % either way ([12000, 1536]
+// 15.5 and 14.9, [24000, 1536] 28.4 and 28.2, [36000, 768] 22.0 and 22.7); [48060, 1536] 61 and 54
+// (rocprofv3, out of cache: 64 and 56), [96120, 768] 60 and 54.  Tanh [3000, 1536] 7.0 and 7.7,
+// [12000, 1536] 18.3 and 17.1; sigmoid 5.4 and 5.2, 13.6 and 12.3.
 #ifndef MBRT_BIAS_WIDE
 #define MBRT_BIAS_WIDE (1ll << 23)
 #endif
 #ifndef MBRT_BIAS_WIDE_GELU
-#define MBRT_BIAS_WIDE_GELU (1ll << 25)
+#define MBRT_BIAS_WIDE_GELU (1ll << 24)
 #endif
 // Pads of 2-byte elements: elements written from which the kernel for whole rows takes them.  Eight of
 // them per thread leave few waves below: [64, 100 -> 200] 2.83 us an element per thread, 3.29 by rows;

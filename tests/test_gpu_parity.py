@@ -536,8 +536,8 @@ def test_bias_act_f32_bias_widths(orc, dev, rows, cols, dt):
 
 # the same at sizes whose f32 bias goes with 16-byte accesses (and, just below, with 8-byte ones): each
 # call over the whole against calls over its two halves, which are below the limit
-@pytest.mark.parametrize("rows,cols,act", [(8193, 1024, 3), (5462, 1544, 4), (8191, 1024, 4), (32769, 1024, 1),
-                                           (21848, 1536, 2)])
+@pytest.mark.parametrize("rows,cols,act", [(8193, 1024, 3), (5462, 1544, 4), (8191, 1024, 4), (16385, 1024, 1),
+                                           (10928, 1536, 2)])
 def test_bias_act_f32_bias_large(dev, rows, cols, act):
     say(f"bias_act f32 bias whole and halves rows={rows} cols={cols} act={act}")
     g = torch.Generator(device="cuda").manual_seed(rows)
