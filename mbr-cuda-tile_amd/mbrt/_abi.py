@@ -1,7 +1,7 @@
 """ctypes declarations of include/mbrt.h.
 
 Loads lib/libmbrt.so from this package's source tree.  There is no fallback: if the
-library is missing, importing raises (build it with `python mbr-cuda-tile_amd/build.py`).
+library is missing, the first call raises (build it with `python mbr-cuda-tile_amd/build.py`).
 """
 from __future__ import annotations
 
