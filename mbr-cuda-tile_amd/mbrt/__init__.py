@@ -56,9 +56,9 @@ def _load_native():
     """The native calls, or the same ones through ctypes where the module built is for another
     Python or torch (or none is)."""
     path = _abi.calls_path(torch.__version__)
-    lib()  # raises where nothing is built
     if path.exists():
         return _abi.load_calls(path)
+    lib()  # raises where nothing is built
     warnings.warn(f"mbrt: {path.name} is not built (run python mbr-cuda-tile_amd/build.py with this Python): "
                   "calls go through ctypes, at about 5 us more each", RuntimeWarning, stacklevel=4)
     from . import _calls
